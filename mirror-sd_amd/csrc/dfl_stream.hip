@@ -87,7 +87,8 @@ DFL_DEV u32x4 norm8(u32x4 xv, float r, u32x4 gv) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     half2_t p = (half2_t){f2h(mul_f16lo_f32(xv[j], r)), f2h(mul_f16hi_f32(xv[j], r))};
-    p = p * __builtin_bit_cast(half2_t, gv[j]);
+    const uint32_t gj = gv[j];   // (bit_cast of the vector element itself reads element 0)
+    p = p * __builtin_bit_cast(half2_t, gj);
     o[j] = __builtin_bit_cast(uint32_t, p);
   }
   return o;
@@ -1284,7 +1285,8 @@ static void launch_t(const StreamArgs& a, const SKPlan& p, hipStream_t st, hipEv
 template <int WT, int EPI, bool NORM, int MTW>
 static void launch_m_w(const StreamArgs& a, const SKPlan& p, hipStream_t st, hipEvent_t e0,
                        hipEvent_t e1) {
-  constexpr int P = (WT == WT_INT8) ? 3 : 4;
+  // (two m-tiles per wave, normed int8: 2, three spill)
+  constexpr int P = WT != WT_INT8 ? 4 : (NORM && MTW > 1 ? 2 : 3);
   const dim3 grid(p.workers), block(64 * (WG_WAVES + 1));
   if (e0 || e1)
     hipExtLaunchKernelGGL((gsk_gemm_m_kernel<WT, EPI, NORM, P, MTW>), grid, block, 0, st, e0, e1,
