@@ -41,7 +41,7 @@ constexpr int ING_MAX = 4096;      // context rows per ingest pass (at most)
 // the context rows (or the tapped layers' rows) where they lie.
 constexpr int SMALL_ING = 64;
 constexpr int MAX_CHUNKS = 64;     // attention key splits
-constexpr int MT_MAX = 8;          // 32-row m-tiles per M-split GEMM launch
+constexpr int MT_MAX = 2;          // 32-row m-tiles per stream-K GEMM launch
 // Stacked blocks of more than STACK_MIN_ROWS rows (batched drafting) are compute-bound: their
 // projections and the lm_head run on the tile GEMM (MFMA, LDS-staged) over the packed weights,
 // with the epilogues in row kernels.
@@ -524,8 +524,8 @@ int dfl_load_head(dfl_ctx* ctx, const uint16_t* final_norm, const uint16_t* embe
 }
 
 // Stream-K GEMM over the M rows of a block: one 32-row m-tile per launch of the
-// single-tile kernel, or up to 8 m-tiles per launch of the M-split kernel (each weight
-// block read once for all of them).  A normed input (gnorm set) takes its 1/rms rows from
+// single-tile kernel, or two per launch of the two-tile kernel (each weight block read
+// once for both).  A normed input (gnorm set) takes its 1/rms rows from
 // the embedding kernel (rn_from_ss false) or from the row sums of squares that the
 // previous RESID GEMM left in sk_ss (rn_from_ss true).
 static int skgemm(dfl_ctx* ctx, int cat, int wt, int epi, const SKPlan& p,
@@ -565,10 +565,9 @@ static int skgemm(dfl_ctx* ctx, int cat, int wt, int epi, const SKPlan& p,
     a.ss_mstride = ss_stride;
     a.gnorm = gnorm;
     a.ws = ctx->sk_ws;
-    // one m-tile: the hybrid plan when it has whole tiles per workgroup; the M-split kernel
-    // and the fused qkv kernel (a Q/K head's two tiles complete together) keep the
-    // contiguous partition
-    a.dp = streamk_launch_dp(p, epi, mt_n > 1);
+    // the hybrid plan when it has whole tiles per workgroup; the fused qkv kernel (a Q/K
+    // head's two tiles complete together) keeps the contiguous partition
+    a.dp = streamk_launch_dp(p, epi, false);
     // test hook of the balanced kernel's bounded work-queue wait (its give-up path), set
     // only through dfl_test_queue_timeout
     a.dyn_test_timeout = p.dyn_static > 0 && ctx->test_queue_timeout;
@@ -591,8 +590,8 @@ static int skgemm(dfl_ctx* ctx, int cat, int wt, int epi, const SKPlan& p,
       a.samp_seed = ctx->call_seed;
       a.samp_row0 = m0;
     }
-    // the balanced kernel (one m-tile) finalises the argmax ids itself
-    const bool fin = ids && keys && p.dyn_static > 0 && n_mt == 1;
+    // the balanced kernel finalises the argmax ids of its rows itself
+    const bool fin = ids && keys && p.dyn_static > 0 && n_mt <= MT_MAX;
     a.ids = fin ? ids : nullptr;
     if (ids_done) *ids_done = fin;
     if (rope) a.rope = *rope;

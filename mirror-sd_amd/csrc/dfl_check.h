@@ -33,7 +33,7 @@ inline const char* check_stream_args(int wt, int epi, bool norm, const StreamArg
     return "null activations";
   }
   if (a.M < 1) return "no activation rows";
-  if (m_split ? (a.MT < 2 || a.MT > 8 || a.M > 32 * a.MT) : (a.M > 32))
+  if (m_split ? (a.MT != 2 || a.M > 32 * a.MT) : (a.M > 32))
     return "activation rows exceed the kernel's m-tiles";
   if (p.workers < 1 || a.seg_cap < 1 || !a.ws || !a.tile_cnt)
     return "missing split-tile workspace";
@@ -78,7 +78,7 @@ inline const char* check_stream_args(int wt, int epi, bool norm, const StreamArg
   if (a.x_zero && epi != EPI_RESID) return "a zero residual (x_zero) is a RESID option";
   if (p.dyn_static > 0 && (!a.dyn_next || !a.err || (a.KB & 1) || epi != EPI_ARGMAX))
     return "balanced plan needs work counters, an error word and an even k-block count";
-  if (a.dp > 0 && ((long long)a.dp * p.workers > a.N / 64 || m_split))
+  if (a.dp > 0 && (long long)a.dp * p.workers > a.N / 64)
     return "hybrid plan with more whole tiles than the matrix has";
   // the fused qkv kernel completes a Q/K head's two tiles together over the contiguous
   // stream-K partition only (its whole-tile loop runs the V-head epilogue)

@@ -51,7 +51,7 @@ struct StreamArgs {
   const half_t* xr_p[MAX_FEATS];
   long long xr_ld;
   int xr_n, xr_h;
-  int MT;                   // M-split kernel: 32-row m-tiles of X (M <= 32 * MT)
+  int MT;                   // two-tile kernel: 32-row m-tiles of X (M <= 32 * MT)
   const float* rnorm;       // NORM: per-row 1/rms of X (used when ss_in is null)
   const float* ss_in;       // NORM: [ss_tiles][32] row sums of squares of X (RESID output)
   int ss_tiles, ss_n;       //       tiles of ss_in, and the row length they sum over
@@ -98,10 +98,9 @@ struct SKPlan {
 };
 // streamk_plan / streamk_plan_balanced (the partition of a matrix over the CUs) are in
 // dfl_sk_plan.h.
-// M-split variant for 2 <= MT <= 8 m-tiles (M <= 256 rows): every weight block is read
-// once for all m-tiles.  X, out, x, ss_*, rnorm, logits, keys point at m-tile 0; m-tile mt
-// is 32*mt rows further (ss blocks ss_mstride floats further).  ws holds
-// [N/64][seg_cap][MT][2048] floats.
+// Variant for MT = 2 m-tiles (33 to 64 rows): every weight block is read once for both.
+// X, out, x, ss_*, rnorm, logits, keys point at m-tile 0; m-tile mt is 32*mt rows further
+// (ss blocks ss_mstride floats further).  ws holds [N/64][seg_cap][MT][2048] floats.
 // Both launchers return false (and launch nothing) for a weight type / epilogue pair
 // they have no kernel for.
 bool launch_streamk_gemm_m(int wt, int epi, bool norm, const StreamArgs& a, const SKPlan& p,

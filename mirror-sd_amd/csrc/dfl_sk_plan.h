@@ -13,8 +13,8 @@ inline SKPlan streamk_plan(int N, int KB, int n_cu) {
   // the largest multiple of the tile count that fits, so every tile is split into the
   // same number of equal k-ranges (no worker straddles two tiles).  With at least one
   // tile per CU, each workgroup also gets dp = tiles / CUs whole tiles, streamed after its
-  // share of the remaining tiles' split units (hybrid plan; the M-split kernel keeps the
-  // contiguous partition, whose slot count is seg_cap).
+  // share of the remaining tiles' split units (hybrid plan; a
+  // launch on the contiguous partition uses seg_cap slots).
   SKPlan p;
   const long long nt = N / 64;
   const long long U = nt * KB;
@@ -49,10 +49,10 @@ inline SKPlan streamk_plan_balanced(int N, int KB, int n_cu) {
   return p;
 }
 
-// Whole tiles per workgroup that one launch of plan p uses.  The hybrid plan (dp > 0) needs
-// the single-tile kernel; the M-split kernel and the fused qkv kernel (EPI_QKROPE: a Q/K
-// head's two tiles complete together, worker counts taken from the contiguous partition)
-// keep the contiguous partition.
+// Whole tiles per workgroup that one launch of plan p uses.  The fused qkv kernel
+// (EPI_QKROPE: a Q/K head's two tiles complete together, worker counts taken from the
+// contiguous partition) and a launch that splits the m-tiles over the waves (m_split; none
+// does any more) keep the contiguous partition.
 inline int streamk_launch_dp(const SKPlan& p, int epi, bool m_split) {
   return (!m_split && epi != EPI_QKROPE) ? p.dp : 0;
 }

@@ -163,12 +163,14 @@ DFL_DEV float rn_from_ss(const float* ss, int tiles, int n, float eps, int lane)
 // reducer wave through LDS slot set (segment & 1), while the next units' loads are already
 // in flight.
 // ---------------------------------------------------------------------------------------
-// XRM (fp16 only): the activations are row-major feature rows (StreamArgs::xr_p) instead of
+// MT: activation m-tiles (32 rows each) multiplied by every weight unit.  Each wave takes its
+// quarter of the units for all of them, so a weight block is loaded and dequantised once.
+// XRM (fp16, one m-tile only): the activations are row-major feature rows (StreamArgs::xr_p) instead of
 // the fragment-layout tile X; lane (m, g) of k-block kb loads X[m][16 kb + 8 g .. + 7], the
 // same eight values its fragment-layout record entry holds.
-template <int WT, bool NORM, int P, bool XRM = false>
+template <int WT, bool NORM, int P, bool XRM = false, int MT = 1>
 DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* rn_lds,
-                          int* ready, float (*red)[WG_WAVES][2048], int* arrived, int* reduced,
+                          int* ready, float (*red)[WG_WAVES][MT * 2048], int* arrived, int* reduced,
                           long long u0, long long u1, long long v0, long long v1, int w,
                           int lane, int& si, const int* abort = nullptr) {
   constexpr int KBK = KTraits<WT>::KBK;
@@ -179,8 +181,10 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
   // activation records: int8 k-block kb = 32 k -> records (kb, 0), (kb, 1), this lane's
   // entry; fp16 k-block kb = 16 k -> record (kb/2, g) at entry m + 32*(kb & 1)
   const u32x4* xf = reinterpret_cast<const u32x4*>(a.X);
+  [[maybe_unused]] const size_t xmt = (size_t)4 * a.ldx;   // 16-byte entries of one m-tile of X
 
-  floatx16 acc0 = (floatx16){}, acc1 = (floatx16){};
+  floatx16 acc[MT][2];
+  static_for<0, MT>([&](auto j) { acc[j][0] = acc[j][1] = (floatx16){}; });
   // si: segments flushed so far by this wave (continues across calls)
   auto flush = [&]() {
     // slot set si & 1 was last used by segment si - 2: wait until it has been reduced (or
@@ -188,16 +192,17 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
     while (__hip_atomic_load(reduced, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < si - 1 &&
            !(abort && __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)))
       __builtin_amdgcn_s_sleep(1);
-    float* dst = red[si & 1][w];
+    static_for<0, MT>([&](auto j) {
+      float* dst = red[si & 1][w] + 2048 * j;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      dst[r * 64 + lane] = acc0[r];
-      dst[1024 + r * 64 + lane] = acc1[r];
-    }
+      for (int r = 0; r < 16; ++r) {
+        dst[r * 64 + lane] = acc[j][0][r];
+        dst[1024 + r * 64 + lane] = acc[j][1][r];
+      }
+      acc[j][0] = acc[j][1] = (floatx16){};
+    });
     if (lane == 0)
       __hip_atomic_fetch_add(&arrived[si & 1], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    acc0 = (floatx16){};
-    acc1 = (floatx16){};
     ++si;
   };
 
@@ -244,7 +249,7 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
     };
     xr_track(ikb);
     struct Stage {
-      u32x4 w0[P], w1[P], x[P][NX];
+      u32x4 w0[P], w1[P], x[P][MT][NX];
       int kb[P], sg[P];
     };
     auto issue = [&](Stage& st) {
@@ -254,16 +259,18 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
         st.w1[s] = load_stream(wp + (size_t)KB * 64);
         st.kb[s] = ikb;
         st.sg[s] = isg;
-        if constexpr (WT == WT_INT8) {
-          st.x[s][0] = xf[(size_t)(2 * ikb) * 64 + lane];
-          st.x[s][NX - 1] = xf[(size_t)(2 * ikb + 1) * 64 + lane];
-        } else if constexpr (XRM) {
-          u32x4 v = {0u, 0u, 0u, 0u};
-          if (m < a.M) v = *reinterpret_cast<const u32x4*>(xr_row + (16 * ikb - xr_k0));
-          st.x[s][0] = v;
-        } else {
-          st.x[s][0] = xf[(size_t)((ikb >> 1) * 2 + g) * 64 + m + 32 * (ikb & 1)];
-        }
+        static_for<0, MT>([&](auto j) {
+          if constexpr (WT == WT_INT8) {
+            st.x[s][j][0] = xf[j * xmt + (size_t)(2 * ikb) * 64 + lane];
+            st.x[s][j][NX - 1] = xf[j * xmt + (size_t)(2 * ikb + 1) * 64 + lane];
+          } else if constexpr (XRM) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (m < a.M) v = *reinterpret_cast<const u32x4*>(xr_row + (16 * ikb - xr_k0));
+            st.x[s][j][0] = v;
+          } else {
+            st.x[s][j][0] = xf[j * xmt + (size_t)((ikb >> 1) * 2 + g) * 64 + m + 32 * (ikb & 1)];
+          }
+        });
         if (++issued < J) {
           if (issued == J1) {   // into the second range
             it = it2;
@@ -281,7 +288,8 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
         }
       });
     };
-    float rn = 1.0f;
+    float rn[MT];
+    static_for<0, MT>([&](auto j) { rn[j] = 1.0f; });
     auto consume = [&](const Stage& st, int base) {
       static_for<0, P>([&](auto s) {
         if (base + (int)s < J) {
@@ -289,26 +297,37 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
             flush();
             ++cs;
           }
-          u32x4 xa = st.x[s][0], xb = st.x[s][NX - 1];
+          u32x4 xa[MT], xb[MT];
+          static_for<0, MT>([&](auto j) {
+            xa[j] = st.x[s][j][0];
+            xb[j] = st.x[s][j][NX - 1];
+          });
           if constexpr (NORM) {
             const int kk = st.kb[s] * KBK + goff;
-            xa = norm8(xa, rn, *reinterpret_cast<const u32x4*>(gsh + kk));
-            if constexpr (NX > 1) xb = norm8(xb, rn, *reinterpret_cast<const u32x4*>(gsh + kk + 8));
-            else xb = xa;
+            const u32x4 ga = *reinterpret_cast<const u32x4*>(gsh + kk);
+            static_for<0, MT>([&](auto j) { xa[j] = norm8(xa[j], rn[j], ga); });
+            if constexpr (NX > 1) {
+              const u32x4 gb = *reinterpret_cast<const u32x4*>(gsh + kk + 8);
+              static_for<0, MT>([&](auto j) { xb[j] = norm8(xb[j], rn[j], gb); });
+            }
           }
           if constexpr (WT == WT_INT8) {
             half8_t lo0, hi0, lo1, hi1;
             dequant_i8x16(st.w0[s], lo0, hi0);
             dequant_i8x16(st.w1[s], lo1, hi1);
-            const half8_t xl = as_half8(xa), xh = as_half8(xb);
-            acc0 = mfma32x32x16(lo0, xl, acc0);
-            acc1 = mfma32x32x16(lo1, xl, acc1);
-            acc0 = mfma32x32x16(hi0, xh, acc0);
-            acc1 = mfma32x32x16(hi1, xh, acc1);
+            static_for<0, MT>([&](auto j) {
+              const half8_t xl = as_half8(xa[j]), xh = as_half8(xb[j]);
+              acc[j][0] = mfma32x32x16(lo0, xl, acc[j][0]);
+              acc[j][1] = mfma32x32x16(lo1, xl, acc[j][1]);
+              acc[j][0] = mfma32x32x16(hi0, xh, acc[j][0]);
+              acc[j][1] = mfma32x32x16(hi1, xh, acc[j][1]);
+            });
           } else {
-            const half8_t xv = as_half8(xa);
-            acc0 = mfma32x32x16(as_half8(st.w0[s]), xv, acc0);
-            acc1 = mfma32x32x16(as_half8(st.w1[s]), xv, acc1);
+            static_for<0, MT>([&](auto j) {
+              const half8_t xv = as_half8(xa[j]);
+              acc[j][0] = mfma32x32x16(as_half8(st.w0[s]), xv, acc[j][0]);
+              acc[j][1] = mfma32x32x16(as_half8(st.w1[s]), xv, acc[j][1]);
+            });
           }
         }
       });
@@ -320,7 +339,7 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
       issue(A);
       issue(B);   // both stages in flight while the reducer's prologue completes
       wait_ready(ready, PRO_DONE);   // gain and 1/rms from the reducer wave's prologue
-      rn = rn_lds[m];
+      static_for<0, MT>([&](auto j) { rn[j] = rn_lds[32 * j + m]; });
     } else {
       issue(A);
     }
@@ -333,6 +352,8 @@ DFL_DEV void stream_range(const StreamArgs& a, const half_t* gsh, const float* r
       __builtin_amdgcn_sched_barrier(0);
       consume(B, base + P);
     }
+  } else if constexpr (NORM && MT > 1) {
+    wait_ready(ready, PRO_DONE);   // the prologue stages its row sums in a slot set
   }
   // the segment of the last unit, then trailing segments without a unit of this wave
   for (; cs < nseg; ++cs) flush();
@@ -343,16 +364,18 @@ DFL_DEV float* ws_slot(const StreamArgs& a, int t, int slot) {
   return a.ws + ((size_t)t * a.seg_cap + slot) * 2048;
 }
 
-// Publishes this worker's partial in slot (t, slot) and bumps counter `cnt` once the
-// stores have completed (agent-coherent); returns the counter's previous value.
-DFL_DEV int publish_partial(const StreamArgs& a, int lane, int t, int slot, int* cnt,
-                            const floatx16& acc0, const floatx16& acc1) {
-  float* mine = ws_slot(a, t, slot);
+// A partial into its workspace slot (agent-coherent stores).
+DFL_DEV void store_partial(float* mine, int lane, const floatx16& acc0, const floatx16& acc1) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     store_agent(mine + r * 64 + lane, acc0[r]);
     store_agent(mine + 1024 + r * 64 + lane, acc1[r]);
   }
+}
+
+// Bumps counter `cnt` once this wave's stores have completed (agent-coherent); returns the
+// counter's previous value.
+DFL_DEV int bump_counter(int* cnt, int lane) {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -361,6 +384,14 @@ DFL_DEV int publish_partial(const StreamArgs& a, int lane, int t, int slot, int*
   prev = __shfl(prev, 0, 64);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   return prev;
+}
+
+// Publishes this worker's partial in slot (t, slot) and bumps counter `cnt`; returns the
+// counter's previous value.
+DFL_DEV int publish_partial(const StreamArgs& a, int lane, int t, int slot, int* cnt,
+                            const floatx16& acc0, const floatx16& acc1) {
+  store_partial(ws_slot(a, t, slot), lane, acc0, acc1);
+  return bump_counter(cnt, lane);
 }
 
 // acc += slots 0 .. count-1 of tile t, in slot order (deterministic sums).  The loads of up to
@@ -587,19 +618,28 @@ DFL_DEV void tile_epilogue(const StreamArgs& a, int lane, int t, const floatx16&
 }
 
 // Norm prologue of the reducer wave: the gain and ss_in are copied to LDS (issued before
-// any streaming wave's weight load), then 1/rms of each activation row goes to rn_s.
-template <int WT>
+// any streaming wave's weight load), then 1/rms of each activation row goes to rn_s.  ss_s
+// holds the ss_in blocks of every m-tile.
+template <int WT, int MT = 1>
 DFL_DEV void reducer_norm_prologue(const StreamArgs& a, int lane, half_t* gsh, float* ss_s,
                                    float* rn_s, int* ready) {
   const int K = a.KB * KTraits<WT>::KBK;
   copy_to_lds(a.gnorm, gsh, K * 2, lane);
-  float rn = 1.0f;
-  if (a.ss_in) copy_to_lds(a.ss_in, ss_s, a.ss_tiles * 32 * 4, lane);
-  else rn = a.rnorm[lane & 31];
+  float rn[MT];
+  static_for<0, MT>([&](auto j) {
+    rn[j] = 1.0f;
+    if (a.ss_in)
+      copy_to_lds(a.ss_in + (size_t)j * a.ss_mstride, ss_s + j * a.ss_tiles * 32,
+                  a.ss_tiles * 32 * 4, lane);
+    else rn[j] = a.rnorm[32 * j + (lane & 31)];
+  });
   if (lane == 0) mark_issued(ready);
-  __builtin_amdgcn_s_waitcnt(0);   // both copies have landed in LDS
-  if (a.ss_in) rn = rn_from_ss(ss_s, a.ss_tiles, a.ss_n, a.eps, lane);
-  if (lane < 32) rn_s[lane] = rn;
+  __builtin_amdgcn_s_waitcnt(0);   // the copies have landed in LDS
+  static_for<0, MT>([&](auto j) {
+    if (a.ss_in)
+      rn[j] = rn_from_ss(ss_s + j * a.ss_tiles * 32, a.ss_tiles, a.ss_n, a.eps, lane);
+    if (lane < 32) rn_s[32 * j + lane] = rn[j];
+  });
   __builtin_amdgcn_s_waitcnt(0);
   if (lane == 0) __hip_atomic_store(ready, PRO_DONE, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
@@ -607,37 +647,89 @@ DFL_DEV void reducer_norm_prologue(const StreamArgs& a, int lane, half_t* gsh, f
 // Reducer wave, segment si (tile t): waits for the 4 streaming waves' partials, sums them
 // in a fixed order, hands the slot set back and completes the tile -- directly when the
 // segment covers it (count == 1), else as worker `slot` of the `count` sharing it.
-DFL_DEV void sum_wave_partials(int lane, float (*red)[WG_WAVES][2048], int* arrived,
-                               int* reduced, int si, floatx16& acc0, floatx16& acc1,
-                               const int* abort = nullptr) {
+DFL_DEV void wait_arrived(int* arrived, int si, const int* abort) {
   while (__hip_atomic_load(&arrived[si & 1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <
              WG_WAVES * ((si >> 1) + 1) &&
          !(abort && __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)))
     __builtin_amdgcn_s_sleep(1);
+}
+// The four waves' partials at src + wave * stride, in wave order.
+DFL_DEV void sum_slot_set(int lane, const float* src, int stride, floatx16& acc0, floatx16& acc1) {
   acc0 = (floatx16){};
   acc1 = (floatx16){};
 #pragma unroll 1
-  for (int j = 0; j < WG_WAVES; ++j) {
-    const float* src = red[si & 1][j];
+  for (int j = 0; j < WG_WAVES; ++j, src += stride) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       acc0[r] += src[r * 64 + lane];
       acc1[r] += src[1024 + r * 64 + lane];
     }
   }
+}
+DFL_DEV void hand_back(int lane, int* reduced, int si) {
   __builtin_amdgcn_s_waitcnt(0);   // slot reads done before the set is handed back
   if (lane == 0) __hip_atomic_store(reduced, si + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+DFL_DEV void sum_wave_partials(int lane, float (*red)[WG_WAVES][2048], int* arrived,
+                               int* reduced, int si, floatx16& acc0, floatx16& acc1,
+                               const int* abort = nullptr) {
+  wait_arrived(arrived, si, abort);
+  sum_slot_set(lane, red[si & 1][0], 2048, acc0, acc1);
+  hand_back(lane, reduced, si);
+}
 
-template <int EPI>
-DFL_DEV void reduce_segment(const StreamArgs& a, int lane, float (*red)[WG_WAVES][2048],
+// The arguments of m-tile mt as seen by tile_epilogue (a 32-row view).
+DFL_DEV StreamArgs mtile_view(const StreamArgs& a, int mt) {
+  StreamArgs v = a;
+  v.M = min(32, a.M - 32 * mt);
+  const size_t rows = (size_t)32 * mt;
+  if (a.out) v.out = a.out + rows * a.ldo;   // STORE rows / SWIGLU AFL tiles (ldo = N/2)
+  if (a.x) v.x = a.x + rows * a.N;           // RESID AFL tiles
+  if (a.ss_part) v.ss_part = a.ss_part + (size_t)mt * a.ss_mstride;
+  if (a.logits) v.logits = a.logits + rows * a.ldl;
+  if (a.keys) v.keys = a.keys + rows;
+  v.samp_row0 = a.samp_row0 + (int)rows;
+  return v;
+}
+
+template <int EPI, int MT = 1>
+DFL_DEV void reduce_segment(const StreamArgs& a, int lane, float (*red)[WG_WAVES][MT * 2048],
                             int* arrived, int* reduced, int si, int t, int slot, int count,
                             const int* abort = nullptr, unsigned long long* key_acc = nullptr) {
-  const EpiIn in = epi_prefetch<EPI>(a, lane, t);   // in flight while the partials arrive
-  floatx16 acc0, acc1;
-  sum_wave_partials(lane, red, arrived, reduced, si, acc0, acc1, abort);
-  const bool complete = count == 1 || finish_split_tile(a, lane, t, slot, count, acc0, acc1);
-  if (complete) tile_epilogue<EPI>(a, lane, t, acc0, acc1, in, key_acc);
+  if constexpr (MT == 1) {
+    const EpiIn in = epi_prefetch<EPI>(a, lane, t);   // in flight while the partials arrive
+    floatx16 acc0, acc1;
+    sum_wave_partials(lane, red, arrived, reduced, si, acc0, acc1, abort);
+    const bool complete = count == 1 || finish_split_tile(a, lane, t, slot, count, acc0, acc1);
+    if (complete) tile_epilogue<EPI>(a, lane, t, acc0, acc1, in, key_acc);
+  } else {
+    // the same steps for every m-tile; a split tile's MT partials lie side by side in its
+    // slot and are published under one count
+    EpiIn in[MT];
+    static_for<0, MT>([&](auto j) { in[j] = epi_prefetch<EPI>(mtile_view(a, j), lane, t); });
+    wait_arrived(arrived, si, abort);
+    floatx16 acc[MT][2];
+    static_for<0, MT>([&](auto j) {
+      sum_slot_set(lane, red[si & 1][0] + 2048 * j, MT * 2048, acc[j][0], acc[j][1]);
+    });
+    hand_back(lane, reduced, si);
+    if (count > 1) {
+      float* tile_ws = a.ws + (size_t)t * a.seg_cap * MT * 2048;
+      static_for<0, MT>([&](auto j) {
+        store_partial(tile_ws + ((size_t)slot * MT + j) * 2048, lane, acc[j][0], acc[j][1]);
+      });
+      if (bump_counter(a.tile_cnt + t, lane) != count - 1) return;
+      static_for<0, MT>([&](auto j) {
+        acc[j][0] = acc[j][1] = (floatx16){};
+        add_slots_at(tile_ws + 2048 * j, MT * 2048, lane, count, acc[j][0], acc[j][1]);
+      });
+      if (lane == 0) a.tile_cnt[t] = 0;   // next use is a later launch
+    }
+    static_for<0, MT>([&](auto j) {
+      tile_epilogue<EPI>(mtile_view(a, j), lane, t, acc[j][0], acc[j][1], in[j],
+                         key_acc ? key_acc + j : nullptr);
+    });
+  }
 }
 
 // Q or K head h of the fused qkv projection, complete: lo = d 0..63 (tile 2h), hi = d
@@ -752,167 +844,13 @@ DFL_DEV void reduce_head(const StreamArgs& a, int lane, float (*red)[WG_WAVES][2
   qk_head_epilogue(a, lane, t0 >> 1, lo0, lo1, hi0, hi1, tb);
 }
 
-// ---------------------------------------------------------------------------------------
-// M-split mode (2 <= MT <= 8 activation m-tiles): streaming wave w owns m-tiles
-// w*MTW .. w*MTW + MTW - 1 and walks every unit of the workgroup range in order, so each
-// weight block is read from HBM once (the other waves hit the cache) and dequantised in
-// registers once per wave for MTW m-tiles.  At each tile end the wave hands its MTW
-// partials to the reducer through LDS slot set (segment & 1).
-// ---------------------------------------------------------------------------------------
-template <int WT, bool NORM, int P, int MTW>
-DFL_DEV void stream_range_m(const StreamArgs& a, const half_t* gsh, const float* rn_lds,
-                            int* ready, float (*red)[WG_WAVES][MTW][2048], int* arrived,
-                            int* reduced, long long u0, long long u1, int w, int lane) {
-  constexpr int KBK = KTraits<WT>::KBK;
-  constexpr int NX = KTraits<WT>::NX;
-  const int m = lane & 31, g = lane >> 5;
-  const int goff = (WT == WT_INT8 ? 16 * g : 8 * g);
-  const int KB = a.KB;
-  const int mt0 = w * MTW;
-  const int nmt = max(0, min(MTW, a.MT - mt0));   // m-tiles of this wave
-  const size_t xstride = (size_t)32 * a.ldx;      // halves from one AFL m-tile to the next
-
-  floatx16 acc[MTW][2];
-#pragma unroll
-  for (int j = 0; j < MTW; ++j) acc[j][0] = acc[j][1] = (floatx16){};
-  int si = 0;
-  auto flush = [&]() {
-    while (__hip_atomic_load(reduced, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < si - 1)
-      __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-    for (int j = 0; j < MTW; ++j) {
-      float* dst = red[si & 1][w][j];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        dst[r * 64 + lane] = acc[j][0][r];
-        dst[1024 + r * 64 + lane] = acc[j][1][r];
-      }
-      acc[j][0] = acc[j][1] = (floatx16){};
-    }
-    if (lane == 0)
-      __hip_atomic_fetch_add(&arrived[si & 1], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    ++si;
-  };
-  const int t_first = (int)(u0 / KB);
-  const int t_last = (int)((u1 - 1) / KB);
-  if (nmt == 0) {   // no m-tile here: hand over zero partials, in step with the others
-    for (int t = t_first; t <= t_last; ++t) flush();
-    return;
-  }
-  const u32x4* xf[MTW];
-#pragma unroll
-  for (int j = 0; j < MTW; ++j)
-    xf[j] = reinterpret_cast<const u32x4*>(a.X + (size_t)(mt0 + min(j, nmt - 1)) * xstride);
-
-  const int J = (int)(u1 - u0);
-  int ct = t_first;
-  int it = t_first, ikb = (int)(u0 - (long long)t_first * KB), issued = 0;
-  struct Stage {
-    u32x4 w0[P], w1[P], x[P][MTW][NX];
-    int kb[P], t[P];
-  };
-  auto issue = [&](Stage& st) {
-    static_for<0, P>([&](auto s) {
-      const uint4* wp = a.W + ((size_t)(2 * it) * KB + ikb) * 64 + lane;
-      st.w0[s] = load_stream(wp);
-      st.w1[s] = load_stream(wp + (size_t)KB * 64);
-      st.kb[s] = ikb;
-      st.t[s] = it;
-#pragma unroll
-      for (int j = 0; j < MTW; ++j) {
-        if constexpr (WT == WT_INT8) {
-          st.x[s][j][0] = xf[j][(size_t)(2 * ikb) * 64 + lane];
-          st.x[s][j][NX - 1] = xf[j][(size_t)(2 * ikb + 1) * 64 + lane];
-        } else {
-          st.x[s][j][0] = xf[j][(size_t)((ikb >> 1) * 2 + g) * 64 + m + 32 * (ikb & 1)];
-        }
-      }
-      if (++issued < J) {
-        if (++ikb == KB) {
-          ikb = 0;
-          ++it;
-        }
-      }
-    });
-  };
-  float rn[MTW];
-#pragma unroll
-  for (int j = 0; j < MTW; ++j) rn[j] = 1.0f;
-  auto consume = [&](const Stage& st, int base) {
-    static_for<0, P>([&](auto s) {
-      if (base + (int)s < J) {
-        while (ct < st.t[s]) {
-          flush();
-          ++ct;
-        }
-        half8_t lo0, hi0, lo1, hi1;
-        if constexpr (WT == WT_INT8) {
-          dequant_i8x16(st.w0[s], lo0, hi0);
-          dequant_i8x16(st.w1[s], lo1, hi1);
-        }
-#pragma unroll
-        for (int j = 0; j < MTW; ++j) {
-          if (j < nmt) {
-            u32x4 xa = st.x[s][j][0], xb = st.x[s][j][NX - 1];
-            if constexpr (NORM) {
-              const int kk = st.kb[s] * KBK + goff;
-              xa = norm8(xa, rn[j], *reinterpret_cast<const u32x4*>(gsh + kk));
-              if constexpr (NX > 1)
-                xb = norm8(xb, rn[j], *reinterpret_cast<const u32x4*>(gsh + kk + 8));
-              else xb = xa;
-            }
-            if constexpr (WT == WT_INT8) {
-              const half8_t xl = as_half8(xa), xh = as_half8(xb);
-              acc[j][0] = mfma32x32x16(lo0, xl, acc[j][0]);
-              acc[j][1] = mfma32x32x16(lo1, xl, acc[j][1]);
-              acc[j][0] = mfma32x32x16(hi0, xh, acc[j][0]);
-              acc[j][1] = mfma32x32x16(hi1, xh, acc[j][1]);
-            } else {
-              const half8_t xv = as_half8(xa);
-              acc[j][0] = mfma32x32x16(as_half8(st.w0[s]), xv, acc[j][0]);
-              acc[j][1] = mfma32x32x16(as_half8(st.w1[s]), xv, acc[j][1]);
-            }
-          }
-        }
-      }
-    });
-  };
-
-  Stage A, B;
-  if constexpr (NORM) {
-    wait_ready(ready, PRO_ISSUED);
-    issue(A);
-    issue(B);   // both stages in flight while the reducer's prologue completes
-    wait_ready(ready, PRO_DONE);
-#pragma unroll
-    for (int j = 0; j < MTW; ++j) rn[j] = rn_lds[(mt0 + min(j, nmt - 1)) * 32 + m];
-  } else {
-    issue(A);
-  }
-  for (int base = 0; base < J; base += 2 * P) {
-    if (!NORM || base > 0) issue(B);
-    __builtin_amdgcn_sched_barrier(0);
-    consume(A, base);
-    if (base + P >= J) break;
-    issue(A);
-    __builtin_amdgcn_sched_barrier(0);
-    consume(B, base + P);
-  }
-  for (int t = ct; t <= t_last; ++t) flush();
-}
-
-// The arguments of m-tile mt as seen by tile_epilogue (a 32-row view).
-DFL_DEV StreamArgs mtile_view(const StreamArgs& a, int mt) {
-  StreamArgs v = a;
-  v.M = min(32, a.M - 32 * mt);
-  const size_t rows = (size_t)32 * mt;
-  if (a.out) v.out = a.out + rows * a.ldo;   // STORE rows / SWIGLU AFL tiles (ldo = N/2)
-  if (a.x) v.x = a.x + rows * a.N;           // RESID AFL tiles
-  if (a.ss_part) v.ss_part = a.ss_part + (size_t)mt * a.ss_mstride;
-  if (a.logits) v.logits = a.logits + rows * a.ldl;
-  if (a.keys) v.keys = a.keys + rows;
-  v.samp_row0 = a.samp_row0 + (int)rows;
-  return v;
+// ARGMAX: the rows' best keys of this workgroup, one atomicMax per row.
+template <int MT>
+DFL_DEV void publish_keys(const StreamArgs& a, int lane, const unsigned long long (&kacc)[MT]) {
+  static_for<0, MT>([&](auto j) {
+    if (a.keys && lane < 32 && 32 * j + lane < a.M && kacc[j])
+      atomicMax(a.keys + 32 * j + lane, kacc[j]);
+  });
 }
 
 }  // namespace
@@ -920,12 +858,16 @@ DFL_DEV StreamArgs mtile_view(const StreamArgs& a, int mt) {
 // ---------------------------------------------------------------------------------------
 // The stream-K kernel: one workgroup per CU, 4 streaming waves + 1 reducer wave.
 // ---------------------------------------------------------------------------------------
-template <int WT, int EPI, bool NORM, int P, bool XRM = false>
-__global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_gemm_kernel(StreamArgs a) {
-  __shared__ float red[2][WG_WAVES][2048];     // partial slots, two sets
-  __shared__ half_t gsh[NORM ? 8192 : 8];
-  __shared__ float ss_s[NORM ? 128 * 32 : 1];  // LDS copy of ss_in (<= 128 tiles)
-  __shared__ float rn_s[32];
+template <int WT, int EPI, bool NORM, int P, bool XRM, int MT>
+DFL_DEV void gsk_gemm_body(const StreamArgs& a) {
+  __shared__ __attribute__((aligned(16))) float red[2][WG_WAVES][MT * 2048];   // partial slots, two sets
+  __shared__ __attribute__((aligned(16))) half_t gsh[NORM ? 8192 : 8];
+  // LDS copy of ss_in (<= 128 tiles); with several m-tiles it goes to the second slot set,
+  // which no wave writes before the prologue is done
+  __shared__ __attribute__((aligned(16))) float ss_own[NORM && MT == 1 ? 128 * 32 : 4];
+  float* ss_s = MT == 1 ? ss_own : red[1][0];
+  static_assert(MT == 1 || MT * 128 * 32 <= WG_WAVES * MT * 2048, "row sums fit a slot set");
+  __shared__ float rn_s[32 * MT];
   // arrived[p]: partials written for segments of parity p (monotonic: a set is rewritten
   // only after its previous segment was reduced); reduced: segments summed so far;
   // ready: norm prologue state (PRO_ISSUED, PRO_DONE)
@@ -957,13 +899,13 @@ __global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_gemm_kernel(StreamArg
 
   if (w < WG_WAVES) {
     int si = 0;
-    stream_range<WT, NORM, P, XRM>(a, gsh, rn_s, &ready, red, arrived, &reduced, u0, u1, v0, v1,
-                                   w, lane, si);
+    stream_range<WT, NORM, P, XRM, MT>(a, gsh, rn_s, &ready, red, arrived, &reduced, u0, u1, v0,
+                                       v1, w, lane, si);
     return;
   }
 
   // ---- reducer wave ----
-  if constexpr (NORM) reducer_norm_prologue<WT>(a, lane, gsh, ss_s, rn_s, &ready);
+  if constexpr (NORM) reducer_norm_prologue<WT, MT>(a, lane, gsh, ss_s, rn_s, &ready);
   [[maybe_unused]] const QkTables qkt{qk_sc, qk_cs, qk_gn};
   if constexpr (EPI == EPI_QKROPE) {   // needed by the first head's epilogue, not before
     copy_to_lds(a.scale, qk_sc, a.N * 2, lane);
@@ -972,8 +914,8 @@ __global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_gemm_kernel(StreamArg
     copy_to_lds(a.rope.k_norm, qk_gn + 128, 256, lane);
   }
   // ARGMAX: each row's best key over the tiles this wave completes, one atomicMax at the end
-  unsigned long long kacc = 0;
-  unsigned long long* ka = EPI == EPI_ARGMAX ? &kacc : nullptr;
+  unsigned long long kacc[MT] = {};
+  unsigned long long* ka = EPI == EPI_ARGMAX ? kacc : nullptr;
   int si = 0;
   for (long long u = u0; u < u1; ++si) {
     const int t = (int)(u / a.KB);
@@ -997,14 +939,30 @@ __global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_gemm_kernel(StreamArg
       first = worker_of(tu0, U, G);
       count = worker_of(tu0 + a.KB - 1, U, G) - first + 1;
     }
-    reduce_segment<EPI>(a, lane, red, arrived, &reduced, si, t, b - first, count, nullptr, ka);
+    reduce_segment<EPI, MT>(a, lane, red, arrived, &reduced, si, t, b - first, count, nullptr, ka);
     u += kbe - kbs;
   }
   for (long long u = v0; u < v1; u += a.KB, ++si)   // whole tiles: local epilogues
-    reduce_segment<EPI>(a, lane, red, arrived, &reduced, si, (int)(u / a.KB), 0, 1, nullptr,
-                        ka);
-  if constexpr (EPI == EPI_ARGMAX)
-    if (a.keys && lane < 32 && lane < a.M && kacc) atomicMax(a.keys + lane, kacc);
+    reduce_segment<EPI, MT>(a, lane, red, arrived, &reduced, si, (int)(u / a.KB), 0, 1, nullptr,
+                            ka);
+  if constexpr (EPI == EPI_ARGMAX) publish_keys<MT>(a, lane, kacc);
+}
+
+template <int WT, int EPI, bool NORM, int P, bool XRM = false>
+__global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_gemm_kernel(StreamArgs a) {
+  gsk_gemm_body<WT, EPI, NORM, P, XRM, 1>(a);
+}
+// Two m-tiles (33 to 64 rows: stacked blocks, long per-step ingests): HBM-bound like the
+// one-tile kernel, every weight byte read and dequantised once for both.  The waves split the
+// units, as with one m-tile, and each multiplies its units with both m-tiles (64 accumulator
+// registers, six int8 units in flight); the earlier split of the m-tiles over the waves left
+// two of the four streaming waves idle.  us per launch, before -> now: 8B-class gate|up at 48
+// rows (100 MB) 106.9 -> 38.4 (2.6 TB/s), qkv (25 MB) 41.0 -> 21.0, o / down 29.1 -> 21.9; 45
+// ingest rows at 27B sizes: fc (262 MB) 81.8 -> 58.5 (4.5 TB/s), all layers' K|V 92.4 -> 30.0.
+// (Three int8 units per stage: four do not fit the 256 registers of a wave.)
+template <int WT, int EPI, bool NORM, int P>
+__global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_gemm_m_kernel(StreamArgs a) {
+  gsk_gemm_body<WT, EPI, NORM, P, false, 2>(a);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1033,12 +991,13 @@ constexpr int DYN_ERR = 4;                // device error bit: a queue wait gave
 // ends normally.
 constexpr int DYN_TEST_SPIN_LIMIT = 256;
 
-template <int WT, int EPI, bool NORM, int P>
-__global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_dyn_kernel(StreamArgs a) {
-  __shared__ float red[2][WG_WAVES][2048];
-  __shared__ half_t gsh[NORM ? 8192 : 8];
-  __shared__ float ss_s[NORM ? 128 * 32 : 1];
-  __shared__ float rn_s[32];
+template <int WT, int EPI, bool NORM, int P, int MT>
+DFL_DEV void gsk_dyn_body(const StreamArgs& a) {
+  __shared__ __attribute__((aligned(16))) float red[2][WG_WAVES][MT * 2048];
+  __shared__ __attribute__((aligned(16))) half_t gsh[NORM ? 8192 : 8];
+  __shared__ __attribute__((aligned(16))) float ss_own[NORM && MT == 1 ? 128 * 32 : 4];
+  float* ss_s = MT == 1 ? ss_own : red[1][0];   // (as in gsk_gemm_body)
+  __shared__ float rn_s[32 * MT];
   __shared__ int arrived[2], reduced, ready;
   __shared__ int q_chunk[4], q_pub;
   // abort: set by a streaming wave whose queue wait gave up; every other wait of the
@@ -1063,9 +1022,9 @@ __global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_dyn_kernel(StreamArgs
   if (w < WG_WAVES) {
     int si = 0;
     if (S > 0)
-      stream_range<WT, NORM, P>(a, gsh, rn_s, &ready, red, arrived, &reduced,
-                                (long long)b * S * KB, (long long)(b + 1) * S * KB, 0, 0, w,
-                                lane, si, &abort);
+      stream_range<WT, NORM, P, false, MT>(a, gsh, rn_s, &ready, red, arrived, &reduced,
+                                           (long long)b * S * KB, (long long)(b + 1) * S * KB, 0,
+                                           0, w, lane, si, &abort);
     const int limit = a.dyn_test_timeout ? DYN_TEST_SPIN_LIMIT : DYN_SPIN_LIMIT;
     for (int k = 0;; ++k) {
       int spins = 0;
@@ -1084,14 +1043,14 @@ __global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_dyn_kernel(StreamArgs
       const int c = q_chunk[k & 3];
       if (c < 0) break;
       const long long c0 = (long long)(T0 + (c >> 1)) * KB + (long long)(c & 1) * half;
-      stream_range<WT, NORM, P>(a, gsh, rn_s, &ready, red, arrived, &reduced, c0, c0 + half, 0,
-                                0, w, lane, si, &abort);
+      stream_range<WT, NORM, P, false, MT>(a, gsh, rn_s, &ready, red, arrived, &reduced, c0,
+                                           c0 + half, 0, 0, w, lane, si, &abort);
     }
     return;
   }
 
   // ---- reducer wave ----
-  if constexpr (NORM) reducer_norm_prologue<WT>(a, lane, gsh, ss_s, rn_s, &ready);
+  if constexpr (NORM) reducer_norm_prologue<WT, MT>(a, lane, gsh, ss_s, rn_s, &ready);
   int n_pub = 0;
   bool exhausted = false;
   auto publish_next = [&]() {
@@ -1112,22 +1071,21 @@ __global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_dyn_kernel(StreamArgs
   int si = 0;
   // ARGMAX: the best key of each row over this workgroup's tiles, one atomicMax per row at
   // the end (one per row and tile contended on the same 32 keys: 8.5 us of the lm_head)
-  unsigned long long kacc = 0;
-  unsigned long long* ka = EPI == EPI_ARGMAX ? &kacc : nullptr;
+  unsigned long long kacc[MT] = {};
+  unsigned long long* ka = EPI == EPI_ARGMAX ? kacc : nullptr;
   for (int i = 0; i < S; ++i, ++si) {
     if (i == S - 1) publish_next();   // entry 0 before the last static segment's wait
-    reduce_segment<EPI>(a, lane, red, arrived, &reduced, si, b * S + i, 0, 1, &abort, ka);
+    reduce_segment<EPI, MT>(a, lane, red, arrived, &reduced, si, b * S + i, 0, 1, &abort, ka);
   }
   if (S == 0) publish_next();
   for (int k = 0;; ++k, ++si) {
     const int c = __shfl(q_chunk[k & 3], 0, 64);   // entry k, published by this wave
     if (c < 0) break;
     publish_next();                   // entry k + 1 before waiting for chunk k
-    reduce_segment<EPI>(a, lane, red, arrived, &reduced, si, T0 + (c >> 1), c & 1, 2, &abort,
-                        ka);
+    reduce_segment<EPI, MT>(a, lane, red, arrived, &reduced, si, T0 + (c >> 1), c & 1, 2, &abort,
+                            ka);
   }
-  if constexpr (EPI == EPI_ARGMAX)
-    if (a.keys && lane < 32 && lane < a.M && kacc) atomicMax(a.keys + lane, kacc);
+  if constexpr (EPI == EPI_ARGMAX) publish_keys<MT>(a, lane, kacc);
   // this workgroup's epilogue atomics and stores are performed before it counts itself
   // finished, so the last one to finish sees every tile's argmax key
   __builtin_amdgcn_s_waitcnt(0);
@@ -1149,110 +1107,13 @@ __global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_dyn_kernel(StreamArgs
   }
 }
 
-// ---------------------------------------------------------------------------------------
-// The M-split stream-K kernel (2 <= MT <= 8): same partition, reducer and completion as
-// gsk_gemm_kernel, with the m-tiles (not the k-blocks) divided among the streaming waves.
-// ---------------------------------------------------------------------------------------
-template <int WT, int EPI, bool NORM, int P, int MTW>
-__global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_gemm_m_kernel(StreamArgs a) {
-  constexpr int KBK = KTraits<WT>::KBK;
-  __shared__ float red[2][WG_WAVES][MTW][2048];
-  __shared__ half_t gsh[NORM ? 8192 : 8];
-  __shared__ float rn_s[32 * WG_WAVES * MTW];
-  __shared__ int arrived[2], reduced, ready;
-
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = gridDim.x;
-  const int b = blockIdx.x;
-  const long long U = (long long)(a.N >> 6) * a.KB;
-  const long long u0 = (long long)b * U / G, u1 = (long long)(b + 1) * U / G;
-  if (u0 >= u1) return;
-  if (threadIdx.x == 0) {
-    arrived[0] = arrived[1] = 0;
-    reduced = 0;
-    ready = 0;
-  }
-  __syncthreads();
-
-  if (w < WG_WAVES) {
-    stream_range_m<WT, NORM, P, MTW>(a, gsh, rn_s, &ready, red, arrived, &reduced, u0, u1, w,
-                                     lane);
-    return;
-  }
-
-  // ---- reducer wave ----
-  if constexpr (NORM) {
-    const int K = a.KB * KBK;
-    copy_to_lds(a.gnorm, gsh, K * 2, lane);
-    if (lane == 0) mark_issued(&ready);
-    for (int mt = 0; mt < a.MT; ++mt) {
-      const float rn = a.ss_in ? rn_from_ss(a.ss_in + (size_t)mt * a.ss_mstride, a.ss_tiles,
-                                            a.ss_n, a.eps, lane)
-                               : a.rnorm[mt * 32 + (lane & 31)];
-      if (lane < 32) rn_s[mt * 32 + lane] = rn;
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    if (lane == 0) __hip_atomic_store(&ready, PRO_DONE, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }
-  int si = 0;
-  for (long long u = u0; u < u1; ++si) {
-    const int t = (int)(u / a.KB);
-    const int kbs = (int)(u - (long long)t * a.KB);
-    const int kbe = (int)min((long long)a.KB, (long long)kbs + (u1 - u));
-    while (__hip_atomic_load(&arrived[si & 1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <
-           WG_WAVES * ((si >> 1) + 1))
-      __builtin_amdgcn_s_sleep(1);
-    const bool whole = (kbs == 0 && kbe == a.KB);
-    int slot = 0, count = 1;
-    if (!whole) {
-      const long long tu0 = (long long)t * a.KB;
-      const int first = worker_of(tu0, U, G);
-      count = worker_of(tu0 + a.KB - 1, U, G) - first + 1;
-      slot = b - first;
-    }
-    // whole tile: epilogue straight from LDS; split tile: publish all m-tile partials,
-    // then the last workgroup to arrive sums them slot by slot
-    for (int mt = 0; mt < a.MT; ++mt) {
-      const float* src = red[si & 1][mt / MTW][mt % MTW];
-      floatx16 acc0, acc1;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        acc0[r] = src[r * 64 + lane];
-        acc1[r] = src[1024 + r * 64 + lane];
-      }
-      if (whole) {
-        tile_epilogue<EPI>(mtile_view(a, mt), lane, t, acc0, acc1);
-      } else {
-        float* mine = a.ws + (((size_t)t * a.seg_cap + slot) * a.MT + mt) * 2048;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          store_agent(mine + r * 64 + lane, acc0[r]);
-          store_agent(mine + 1024 + r * 64 + lane, acc1[r]);
-        }
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0);   // slot reads (and partial stores) done
-    if (lane == 0) __hip_atomic_store(&reduced, si + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (!whole) {
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      int prev = 0;
-      if (lane == 0)
-        prev = __hip_atomic_fetch_add(a.tile_cnt + t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      prev = __shfl(prev, 0, 64);
-      if (prev == count - 1) {
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        for (int mt = 0; mt < a.MT; ++mt) {
-          floatx16 acc0 = (floatx16){}, acc1 = (floatx16){};
-          add_slots_at(a.ws + ((size_t)t * a.seg_cap * a.MT + mt) * 2048, (size_t)a.MT * 2048,
-                       lane, count, acc0, acc1);
-          tile_epilogue<EPI>(mtile_view(a, mt), lane, t, acc0, acc1);
-        }
-        if (lane == 0) a.tile_cnt[t] = 0;   // next use is a later launch
-      }
-    }
-    u += kbe - kbs;
-  }
+template <int WT, int EPI, bool NORM, int P>
+__global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_dyn_kernel(StreamArgs a) {
+  gsk_dyn_body<WT, EPI, NORM, P, 1>(a);
+}
+template <int WT, int EPI, bool NORM, int P>
+__global__ __launch_bounds__(64 * (WG_WAVES + 1)) void gsk_dyn_m_kernel(StreamArgs a) {
+  gsk_dyn_body<WT, EPI, NORM, P, 2>(a);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1282,25 +1143,16 @@ static void launch_t(const StreamArgs& a, const SKPlan& p, hipStream_t st, hipEv
     hipLaunchKernelGGL((gsk_gemm_kernel<WT, EPI, NORM, 4, XRM>), grid, block, 0, st, a);
 }
 
-template <int WT, int EPI, bool NORM, int MTW>
-static void launch_m_w(const StreamArgs& a, const SKPlan& p, hipStream_t st, hipEvent_t e0,
-                       hipEvent_t e1) {
-  // (two m-tiles per wave, normed int8: 2, three spill)
-  constexpr int P = WT != WT_INT8 ? 4 : (NORM && MTW > 1 ? 2 : 3);
-  const dim3 grid(p.workers), block(64 * (WG_WAVES + 1));
-  if (e0 || e1)
-    hipExtLaunchKernelGGL((gsk_gemm_m_kernel<WT, EPI, NORM, P, MTW>), grid, block, 0, st, e0, e1,
-                          0, a);
-  else
-    hipLaunchKernelGGL((gsk_gemm_m_kernel<WT, EPI, NORM, P, MTW>), grid, block, 0, st, a);
-}
-
-// One m-tile per streaming wave up to 4 m-tiles, two up to 8.
 template <int WT, int EPI, bool NORM>
 static void launch_m_t(const StreamArgs& a, const SKPlan& p, hipStream_t st, hipEvent_t e0,
                        hipEvent_t e1) {
-  if (a.MT <= WG_WAVES) launch_m_w<WT, EPI, NORM, 1>(a, p, st, e0, e1);
-  else launch_m_w<WT, EPI, NORM, 2>(a, p, st, e0, e1);
+  constexpr int P = (WT == WT_INT8) ? 3 : 4;
+  const dim3 grid(p.workers), block(64 * (WG_WAVES + 1));
+  auto* kernel = gsk_gemm_m_kernel<WT, EPI, NORM, P>;
+  if constexpr (WT == WT_F16 && EPI == EPI_ARGMAX)
+    if (p.dyn_static > 0) kernel = gsk_dyn_m_kernel<WT, EPI, NORM, P>;
+  if (e0 || e1) hipExtLaunchKernelGGL(kernel, grid, block, 0, st, e0, e1, 0, a);
+  else hipLaunchKernelGGL(kernel, grid, block, 0, st, a);
 }
 
 bool launch_streamk_gemm_m(int wt, int epi, bool norm, const StreamArgs& a, const SKPlan& p,

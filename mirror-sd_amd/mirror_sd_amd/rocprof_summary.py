@@ -38,7 +38,7 @@ GROUPS = [
     ("o / down (RESID)", r"gsk_gemm_kernel<0, 4, false, 4, false>"),
     ("gate|up (SWIGLU, norm-on-load)", r"gsk_gemm_kernel<0, 1, true, 4, false>"),
     ("lm_head (fp16, ARGMAX, norm-on-load)", r"gsk_(gemm_kernel<1, 2, true, 4, false|dyn_kernel<1, 2, true, 4)>"),
-    ("M-split stream-K (stacked rows up to 64)", r"gsk_gemm_m_kernel"),
+    ("two-m-tile stream-K (33 to 64 rows)", r"gsk_(gemm|dyn)_m_kernel"),
     ("per-step ingest fc (fp16, zero-residual RESID: rows + row sums), up to 16 rows read in "
      "place", r"gsk_gemm_kernel<1, 4, false, 4, true>"),
     ("per-step ingest fc, rows gathered into fragment layout first (17-32, or unaligned)",

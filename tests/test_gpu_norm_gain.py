@@ -25,13 +25,17 @@ def _weights(cfg):
     return t
 
 
-@pytest.mark.parametrize("n_seq,block,ctx", [(1, 8, 5),      # one m-tile, ingest of 5 rows
-                                             (1, 8, 40),     # ingest of two m-tiles
-                                             (2, 20, 40),    # 40 stacked rows
-                                             (3, 32, 70)])   # 96 rows, prompt-sized ingest
-def test_column_dependent_norm_gains_match_oracle(n_seq, block, ctx):
+@pytest.mark.parametrize("n_seq,block,ctx,vocab", [
+    (1, 8, 5, 1024),        # one m-tile, ingest of 5 rows
+    (1, 33, 33, 1024),      # two m-tiles with one row in the second, block and ingest
+    (2, 20, 40, 1024),      # 40 stacked rows
+    (2, 32, 64, 33024),     # two whole m-tiles; a vocabulary that takes the balanced lm_head
+    (3, 15, 45, 33024),     # 45 of 64 rows there
+    (3, 32, 70, 1024)])     # 96 rows, prompt-sized ingest
+def test_column_dependent_norm_gains_match_oracle(n_seq, block, ctx, vocab):
     from mirror_sd_amd.dflash import DFlashDraftModel
     cfg = workload("tiny").cfg
+    cfg.vocab_size = vocab
     t = _weights(cfg)
     W = O.OracleWeights(cfg, t)
     inps = synth.make_batch_inputs_numpy(cfg, block, (ctx,) * n_seq, seed=32)
@@ -40,8 +44,10 @@ def test_column_dependent_norm_gains_match_oracle(n_seq, block, ctx):
     for i, inp in enumerate(inps):
         m.ingest_seq(i, torch.from_numpy(inp["target_hidden"]))
     ids = torch.from_numpy(np.stack([inp["ids"] for inp in inps]))
-    _, logits, hidden = m.draft_batch(ids=ids, return_logits=True, return_hidden=True)
-    torch.cuda.synchronize()
+    for _ in range(2):   # the second call meets the counters and keys that the first re-armed
+        got, logits, hidden = m.draft_batch(ids=ids, return_logits=True, return_hidden=True)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(got.cpu().numpy(), logits.argmax(-1).cpu().numpy())
     for i, inp in enumerate(inps):
         h_ref, lg_ref, _ = O.draft_block(W, inp["ids"], inp["target_hidden"], fp16=True)
         assert_close_fp16(hidden[i].float().cpu().numpy(), h_ref, what=f"sequence {i} hidden")
