@@ -205,7 +205,7 @@ int dfl_embed_block(dfl_ctx* ctx, const int32_t* ids, int32_t B, const void* cor
  * table embed [Vemb][H] fp16 (16-byte aligned rows, H % 8 == 0) and a device word err_flags
  * that receives the same error bits as dfl_device_errors (OR'ed in; bit 0 a token id outside
  * [0, Vemb), bit 1 soft-anchor logits without a single number).  Other arguments, checks and
- * results as dfl_embed_block.  The soft anchor's top-k candidates go to a fixed 4 KiB device
+ * results as dfl_embed_block.  The soft anchor's top-k candidates go to a fixed 16 KiB device
  * array of the library (64 scan workgroups x 8 keys, one copy per GPU, held until the process
  * ends), so the call allocates nothing; concurrent calls on one GPU share that array and
  * race, so a caller serialises them (one stream, or events between streams). */

@@ -331,7 +331,7 @@ int dfl_create(const dfl_config* cfg, dfl_ctx** out) {
       (r = x->alloc(&x->Op, (size_t)MAX_CHUNKS * x->NH * Bm * 128)) ||
       (r = x->alloc(&x->Ml, (size_t)MAX_CHUNKS * x->NH * Bm * 2)) ||
       (r = x->alloc(&x->keys, Bm, true)) || (r = x->alloc(&x->err, 1, true)) ||
-      (r = x->alloc(&x->sa_cand, (size_t)SA_BLOCKS * SA_TOPK_MAX))) {
+      (r = x->alloc(&x->sa_cand, (size_t)SA_LISTS * SA_TOPK_MAX))) {
     delete x;
     return r;
   }
@@ -1417,7 +1417,7 @@ int dfl_embed_block(dfl_ctx* ctx, const int32_t* ids, int32_t B, const void* cor
 // Host code uses the per-device address from hipGetSymbolAddress, never the array's name.
 namespace {
 constexpr int NOALLOC_MAX_DEVICES = 64;
-static __device__ __align__(256) unsigned long long scratch[SA_BLOCKS * SA_TOPK_MAX];
+static __device__ __align__(256) unsigned long long scratch[SA_LISTS * SA_TOPK_MAX];
 std::mutex g_scratch_mu;
 unsigned long long* g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
 
@@ -1461,7 +1461,7 @@ int dfl_embed_block_noalloc(const int32_t* ids, int32_t B, const uint16_t* embed
     if (top_k < 1 || top_k > SA_TOPK_MAX)
       return fail(DFL_EINVAL, "dfl_embed_block_noalloc: top_k must be in [1, " +
                                   std::to_string(SA_TOPK_MAX) + "] (the fixed candidate array "
-                                  "holds 64 x 8 keys)");
+                                  "holds 256 x 8 keys)");
     if (V < top_k || V > Vemb)
       return fail(DFL_EINVAL, "dfl_embed_block_noalloc: logits length must be in [top_k, Vemb]");
   }
