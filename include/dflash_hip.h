@@ -93,6 +93,11 @@ int dfl_load_head(dfl_ctx* ctx, const uint16_t* final_norm, const uint16_t* embe
  * offset .. offset+C-1 -- the context half of Qwen3DFlashAttention, dflash.py:287-308;
  * `_compute_context`, ane_model.py:632-637).  target_hidden [C][n_target_feat*H] fp16. */
 int dfl_ingest_context(dfl_ctx* ctx, const uint16_t* target_hidden, int32_t C, void* stream);
+/* The same for sequences 0 .. n_seq-1 in lockstep, C rows each: target_hidden
+ * [n_seq][C][n_target_feat*H].  Short steps of several sequences share one pass over the
+ * fc and K/V weights; each sequence's rows are those of its own dfl_ingest_context call. */
+int dfl_ingest_batch(dfl_ctx* ctx, int32_t n_seq, const uint16_t* target_hidden, int32_t C,
+                     void* stream);
 /* Same for context rows that are already fused ([C][H] fp16): skips fc + hidden_norm. */
 int dfl_ingest_fused(dfl_ctx* ctx, const uint16_t* ctx_hidden, int32_t C, void* stream);
 

@@ -771,8 +771,11 @@ static int ingest_kv_rows(dfl_ctx* ctx, const half_t* xa, int rows, int r0, hipS
 // as it loads those rows (norm-on-load, 1/rms from the fc's row sums; the Linear's scale
 // and fp16 rounding in its epilogue) and k_norm + RoPE into the cache.  The arithmetic of
 // the prompt-sized path (fp32 accumulation, the same rounding points).
-static int ingest_small(dfl_ctx* ctx, const half_t* in, int C, bool fused, const FeatPtrs* feats,
-                        hipStream_t st) {
+// Sequences seq0 .. seq0 + n_seq - 1 take Cs rows each, stacked sequence-major (at most
+// SMALL_ING in all): the fc and the K|V weights are read once for the group.
+static int ingest_small(dfl_ctx* ctx, int seq0, int n_seq, const half_t* in, int Cs, bool fused,
+                        const FeatPtrs* feats, hipStream_t st) {
+  const int C = n_seq * Cs;
   const int H = ctx->H, NH = ctx->NH, NKV = ctx->NKV, Nkv = 2 * NKV * 128;
   FeatPtrs f{};
   if (feats) {
@@ -805,21 +808,23 @@ static int ingest_small(dfl_ctx* ctx, const half_t* in, int C, bool fused, const
   }
   // the K|V rows of all active layers in one GEMM (the all-layer matrix; hidden_norm on
   // load unless the rows came fused), then k_norm + RoPE and the cache writes for up to
-  // SEQ_MAX layers per launch
+  // SEQ_MAX layers x sequences per launch
   const int KB = H / 32;
   const int Nall = ctx->active * Nkv;
   DFL_TRY(skgemm(ctx, P_INGEST_KV, WT_INT8, EPI_STORE, streamk_plan(Nall, KB, ctx->n_cu),
                  ctx->w_kv_all, ctx->s_kv_all, Nall, KB, xsrc, H, C,
                  fused ? nullptr : ctx->hidden_norm, !fused, ctx->si_kv, Nall, nullptr, nullptr,
                  nullptr, st));
-  for (int l0 = 0; l0 < ctx->active; l0 += SEQ_MAX) {
-    const int nl = std::min(SEQ_MAX, ctx->active - l0);
+  const int lmax = std::max(1, SEQ_MAX / n_seq);
+  for (int l0 = 0; l0 < ctx->active; l0 += lmax) {
+    const int nl = std::min(lmax, ctx->active - l0);
     QKRopeArgs q{};
     q.qkv16 = ctx->si_kv + (size_t)l0 * Nkv;
-    q.M = C;
+    q.M = Cs;
     q.N = Nall;
-    q.n_seq = nl;
+    q.n_seq = nl * n_seq;
     q.layer_cols = Nkv;
+    q.layer_seqs = n_seq;
     q.col_slot0 = NH;
     q.slot0 = NH;
     q.n_slots = 2 * NKV;
@@ -832,15 +837,16 @@ static int ingest_small(dfl_ctx* ctx, const half_t* in, int C, bool fused, const
     q.inv_freq = ctx->rope_freqs();
     q.Q = nullptr;   // (a per-step call's few rows compute their angles in place: an angle
     q.cap = ctx->cap;   // table would cost one more launch than it saves)
-    for (int i = 0; i < nl; ++i) {
-      const Layer& L = ctx->layers[l0 + i];
+    for (int i = 0; i < nl * n_seq; ++i) {
+      const Layer& L = ctx->layers[l0 + i / n_seq];
+      const int sidx = seq0 + i % n_seq;
       q.k_norm_s[i] = L.k_norm;
-      rope_seq(ctx, ctx->cur, L, ctx->sq().offset, C, q.sq[i]);
+      rope_seq(ctx, sidx, L, ctx->seqs[sidx].offset, Cs, q.sq[i]);
     }
     ProfScope ps(ctx, P_INGEST_KV, 0, st);
     DFL_TRY(qk_rope(q, st));
   }
-  ctx->sq().append(C);
+  for (int i = 0; i < n_seq; ++i) ctx->seqs[seq0 + i].append(Cs);
   return DFL_OK;
 }
 
@@ -863,7 +869,7 @@ static int ingest(dfl_ctx* ctx, const uint16_t* src, int C, bool fused, void* st
   // per-step context rows: stream-K kernels (any alignment: the rows are gathered into
   // fragment layout first)
   if (C > 0 && C <= SMALL_ING && (fused || ctx->w_fc_pk)) {
-    DFL_TRY(ingest_small(ctx, in, C, fused, feats, st));
+    DFL_TRY(ingest_small(ctx, ctx->cur, 1, in, C, fused, feats, st));
     DFL_TRY(check_launch("ingest"));
     ctx->sq().offset += C;
     return DFL_OK;
@@ -915,6 +921,47 @@ static int ingest(dfl_ctx* ctx, const uint16_t* src, int C, bool fused, void* st
 
 int dfl_ingest_context(dfl_ctx* ctx, const uint16_t* target_hidden, int32_t C, void* stream) {
   return ingest(ctx, target_hidden, C, false, stream);
+}
+
+int dfl_ingest_batch(dfl_ctx* ctx, int32_t n_seq, const uint16_t* target_hidden, int32_t C,
+                     void* stream) {
+  const std::string w = "dfl_ingest_batch";
+  if (!ctx || (!target_hidden && C > 0)) return fail(DFL_EINVAL, w + ": null argument");
+  if (n_seq < 1 || n_seq > ctx->S)
+    return fail(DFL_ERANGE, w + ": n_seq must be in [1, max_seqs=" + std::to_string(ctx->S) + "]");
+  if (C < 0) return fail(DFL_EINVAL, w + ": negative row count");
+  for (int i = 0; i < n_seq; ++i)
+    if (!ctx->seqs[i].window && (long long)ctx->seqs[i].len + C > ctx->cfg.max_ctx)
+      return fail(DFL_ERANGE, w + ": context rows " + std::to_string(ctx->seqs[i].len + C) +
+                                  " of sequence " + std::to_string(i) + " exceed max_ctx " +
+                                  std::to_string(ctx->cfg.max_ctx));
+  DFL_TRY(layers_ready(ctx, "dfl_ingest_batch"));
+  if (!ctx->fc_loaded) return fail(DFL_ESTATE, w + ": fc not loaded");
+  const size_t seq_elems = (size_t)C * ctx->NF * ctx->H;
+  // Groups of sequences whose rows fit one per-step ingest share its launches (the fc alone
+  // reads 2 * NF * H^2 bytes of weights); a longer step ingests sequence by sequence.
+  const int per = C > 0 ? std::min(SEQ_MAX, SMALL_ING / C) : 0;
+  for (int s0 = 0; s0 < n_seq;) {
+    if (per >= 2) {
+      const int n = std::min(per, n_seq - s0);
+      DFL_TRY(ingest_small(ctx, s0, n, reinterpret_cast<const half_t*>(target_hidden) + s0 * seq_elems,
+                           C, false, nullptr, (hipStream_t)stream));
+      DFL_TRY(check_launch(w.c_str()));
+      for (int i = s0; i < s0 + n; ++i) {
+        ctx->seqs[i].last_block = 0;
+        ctx->seqs[i].offset += C;
+      }
+      s0 += n;
+    } else {
+      const int cur = ctx->cur;
+      ctx->cur = s0;
+      const int r = ingest(ctx, target_hidden + s0 * seq_elems, C, false, stream);
+      ctx->cur = cur;
+      if (r != DFL_OK) return r;
+      ++s0;
+    }
+  }
+  return DFL_OK;
 }
 
 int dfl_ingest_fused(dfl_ctx* ctx, const uint16_t* ctx_hidden, int32_t C, void* stream) {

@@ -95,8 +95,11 @@ inline const char* check_qk_rope_args(const QKRopeArgs& a) {
     return "head slots outside the q|k|v heads";
   if (a.layer_cols) {
     if (a.slot0 < a.NH) return "layer mode takes K|V rows only";
+    const int ls = a.layer_seqs > 1 ? a.layer_seqs : 1;
+    if (a.n_seq % ls) return "a layer without an entry for every sequence";
+    if (ls > 1 && a.cs) return "one angle table for several sequences";
     if ((long long)(a.slot0 + a.n_slots - a.col_slot0) * 128 > a.layer_cols ||
-        (long long)a.n_seq * a.layer_cols > a.N)
+        (long long)(a.n_seq / ls) * a.layer_cols > a.N)
       return "slots past the row width";
     for (int s = 0; s < a.n_seq; ++s)
       if (!a.k_norm_s[s]) return "layer mode without a per-layer k_norm";

@@ -258,8 +258,11 @@ struct QKRopeArgs {
   RopeSeq sq[SEQ_MAX];
   // layer mode (layer_cols > 0): the entries are layers of one sequence sharing the rows;
   // entry s reads columns [s * layer_cols, ...) of each row (N is the row stride) and uses
-  // the k_norm gain k_norm_s[s]
+  // the k_norm gain k_norm_s[s].  With layer_seqs > 1 the entries are layers x sequences:
+  // entry s is layer s / layer_seqs of sequence s % layer_seqs, whose rows follow those of
+  // the sequences before it
   int layer_cols;
+  int layer_seqs;
   const half_t* k_norm_s[SEQ_MAX];
 };
 // -1: a ring row that a later row of the same launch overwrites (more than ring_W ring

@@ -308,8 +308,10 @@ __host__ __device__ inline QkRopeGrid qk_rope_grid(const QKRopeArgs& a) {
 
 // Column of slot `slot`, element 0, and the row index of row m in the projection rows.
 DFL_DEV void qk_rope_src(const QKRopeArgs& a, int sidx, int m, int slot, size_t& row, int& c0) {
-  row = a.layer_cols ? (size_t)m : (size_t)sidx * a.M + m;
-  c0 = (a.layer_cols ? sidx * a.layer_cols : 0) + (slot - a.col_slot0) * 128;
+  const int ls = a.layer_seqs > 1 ? a.layer_seqs : 1;
+  const int layer = a.layer_cols ? sidx / ls : 0;
+  row = (size_t)(a.layer_cols ? sidx - layer * ls : sidx) * a.M + m;
+  c0 = layer * a.layer_cols + (slot - a.col_slot0) * 128;
 }
 
 // Projection values (fp16 Linear output, as float) of row `row`, columns c .. c+E-1 (c % E ==

@@ -47,6 +47,7 @@ SIGNATURES = {
     "dfl_load_fc": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p]),
     "dfl_load_head": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "dfl_ingest_context": (c_int32, [c_void_p, c_void_p, c_int32, c_void_p]),
+    "dfl_ingest_batch": (c_int32, [c_void_p, c_int32, c_void_p, c_int32, c_void_p]),
     "dfl_ingest_fused": (c_int32, [c_void_p, c_void_p, c_int32, c_void_p]),
     "dfl_ingest_features": (c_int32, [c_void_p, ctypes.POINTER(c_void_p), c_int32,
                                       ctypes.c_int64, c_int32, c_void_p]),

@@ -521,6 +521,21 @@ class DFlashDraftModel:
         self._keep["ingest_src"] = th   # keep alive until the stream passes it
         return C
 
+    def _ingest_seqs(self, target_hidden):
+        """Context rows [n_seq, C, nf*H] of sequences 0 .. n_seq-1 (dfl_ingest_batch)."""
+        import torch
+        th = target_hidden.to(self.device, torch.float16).contiguous()
+        n_seq, C = th.shape[0], th.shape[1]
+        if C == 0:
+            return 0
+        if th.shape[2] != self.n_feat * self.config.hidden_size:
+            raise ValueError(f"target_hidden must be [C, {self.n_feat * self.config.hidden_size}],"
+                             f" got {tuple(th.shape[1:])}")
+        _lib.check(self._L.dfl_ingest_batch(self._ctx, n_seq, th.data_ptr(), C, self._stream()),
+                   "dfl_ingest_batch")
+        self._keep["ingest_src"] = th   # keep alive until the stream passes it
+        return C
+
     def _draft(self, noise=None, ids=None, want_hidden=True, want_prenorm=False,
                want_logits=False, want_ids=False):
         import torch
@@ -574,18 +589,12 @@ class DFlashDraftModel:
             cache = list(cache)[:self.num_draft_layers]
             self._sync_cache(cache, n_seq=B_)
         self._batch = B_
-        C = 0
-        for b in range(B_):
-            if b:
+        if cache is None:
+            for b in range(B_):
                 self.select_seq(b)
-            try:
-                if cache is None:
-                    _lib.check(self._L.dfl_cache_reset(self._ctx), "dfl_cache_reset")
-                th = target_hidden if B_ == 1 else target_hidden[b]
-                C = self._ingest(th)
-            finally:
-                if b:
-                    self.select_seq(0)
+                _lib.check(self._L.dfl_cache_reset(self._ctx), "dfl_cache_reset")
+            self.select_seq(0)
+        C = self._ingest(target_hidden) if B_ == 1 else self._ingest_seqs(target_hidden)
         if cache is None:
             self._gen += 1
         if B_ == 1:
