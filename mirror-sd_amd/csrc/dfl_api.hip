@@ -625,24 +625,29 @@ static int block_attention(const AttnArgs& at, hipStream_t st) {
 // (the TileArgs outputs e), its argument checks reported as DFL_EINVAL.
 // Split-K (F32 and RESID epilogues of stacked blocks, when the plan finds it faster): the
 // GEMM writes fp32 planes into tile_ws and launch_tile_reduce applies the epilogue.
+// chains (optional): the accumulation chains of the shapes to plan with.
 // n_parts (ARGMAX): receives the number of partial key rows written (one per wave column).
-// like_n (optional): plan with the tile shape the product of like_n columns would have, so
-// that a product stacked over several such (the all-layer K|V ingest) sums every element
-// exactly as the single one does.
+// planes (F32, optional): the caller sums the planes itself: with ws the product may split
+// into planes [splits][M][N] there, and receives the factor (1: written to e.Y); without ws it
+// does not split.
+struct TilePlanes {
+  float* ws;
+  size_t floats;
+  int splits;
+};
 static int tgemm(dfl_ctx* ctx, int cat, int wt, int epi, const uint4* W, int N, int K,
                  const half_t* X, int M, const TileArgs& e, hipStream_t st,
-                 int* n_parts = nullptr, int like_n = 0) {
-  const bool split_ok = (epi == TG_F32 || epi == TG_RESID) && ctx->tile_ws && M <= ctx->RM &&
-                        !like_n;
+                 int* n_parts = nullptr, TilePlanes* planes = nullptr, int chains = 0) {
+  const bool split_ok = planes ? planes->ws != nullptr
+                               : (epi == TG_F32 || epi == TG_RESID) && ctx->tile_ws && M <= ctx->RM;
+  float* ws = planes ? planes->ws : ctx->tile_ws;
+  const size_t ws_floats = planes ? planes->floats : ctx->tile_ws_floats;
   // re-tiled last rounds for the epilogues whose outputs do not depend on the tile shape
   // (the ARGMAX keys are per wave column)
   const bool retile = epi != TG_ARGMAX;
-  TilePlan like{};
-  if (like_n) like = tile_plan(M, like_n, K, wt, ctx->n_cu, epi == TG_SWIGLU);
-  TilePlan p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, split_ok, retile,
-                         like_n ? &like : nullptr);
-  if (p.splits > 1 && (size_t)p.splits * M * N > ctx->tile_ws_floats)   // planes do not fit
-    p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, false, retile);
+  TilePlan p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, split_ok, retile, chains);
+  if (p.splits > 1 && (size_t)p.splits * M * N > ws_floats)   // planes do not fit
+    p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, false, retile, chains);
   if (n_parts) *n_parts = N / (32 * p.rbw);
   TileArgs a = e;
   a.W = W;
@@ -662,23 +667,25 @@ static int tgemm(dfl_ctx* ctx, int cat, int wt, int epi, const uint4* W, int N, 
     g.K = K;
     g.X = X;
     g.M = M;
-    g.Y = ctx->tile_ws;
+    g.Y = ws;
     g.ldy = N;
   }
   const int gepi = p.splits > 1 ? TG_F32 : epi;
   if (const char* why = check_tile_args(wt, gepi, g, p))
     return fail(DFL_EINVAL, std::string("tile GEMM launch refused: ") + why);
-  if (p.splits > 1)
-    if (const char* why = check_tile_reduce_args(epi, a, ctx->tile_ws, p.splits))
+  if (planes) planes->splits = p.splits;
+  const bool reduce = p.splits > 1 && !planes;
+  if (reduce)
+    if (const char* why = check_tile_reduce_args(epi, a, ws, p.splits))
       return fail(DFL_EINVAL, std::string("tile GEMM reduction refused: ") + why);
   if (tile_lds_bytes(wt, p) > (size_t)ctx->lds_max)
     return fail(DFL_EINVAL, "tile GEMM: the device's LDS per workgroup is too small");
   const long long wbytes = (long long)N * K * (wt == WT_INT8 ? 1 : 2);
   // the attached events span the GEMM and, when split, its reduction
   ProfScope ps(ctx, cat, wbytes, st, /*attached=*/true);
-  if (!launch_tile_gemm(wt, gepi, g, p, st, ps.start(), p.splits > 1 ? nullptr : ps.stop()))
+  if (!launch_tile_gemm(wt, gepi, g, p, st, ps.start(), reduce ? nullptr : ps.stop()))
     return fail(DFL_EINVAL, "no tile GEMM kernel for this shape and epilogue");
-  if (p.splits > 1 && !launch_tile_reduce(epi, a, ctx->tile_ws, p.splits, st, ps.stop()))
+  if (reduce && !launch_tile_reduce(epi, a, ws, p.splits, st, ps.stop()))
     return fail(DFL_EINVAL, "tile GEMM reduction refused");
   return DFL_OK;
 }
@@ -728,8 +735,11 @@ static int ingest_kv_rows(dfl_ctx* ctx, const half_t* xa, int rows, int r0, hipS
     launch_rope_table(rows, ctx->sq().offset + r0, std::log2(ctx->cfg.rope_theta),
                       ctx->rope_freqs(), ctx->ing_cs, st);
   }
+  // one layer's accumulation chains and no split: the same sums at any number of layers
+  TilePlanes whole{};
+  const TilePlan one = tile_plan(rows, Nkv, H, WT_INT8, ctx->n_cu);
   DFL_TRY(tgemm(ctx, P_INGEST_KV, WT_INT8, TG_F32, ctx->w_kv_all, Nall, H, xa, rows,
-                tile_f32(ctx->kv32, Nall), st, nullptr, /*like_n=*/Nkv));
+                tile_f32(ctx->kv32, Nall), st, nullptr, &whole, tile_chains(WT_INT8, one.mtw, one.rbw)));
   for (int l0 = 0; l0 < ctx->active; l0 += SEQ_MAX) {
     const int nl = std::min(SEQ_MAX, ctx->active - l0);
     QKRopeArgs q{};
@@ -904,11 +914,15 @@ static int ingest(dfl_ctx* ctx, const uint16_t* src, int C, bool fused, void* st
         ProfScope ps(ctx, P_INGEST_FC, 0, st);
         launch_feats_to_afl(f, rows, H, ctx->xf, st);
       }
+      // Few rows leave CUs without a tile: the product may then split its long K into fp32
+      // planes, in the K|V rows' buffer (free until the K|V product), which the norm sums
+      // (300 rows at 27B sizes: 117 us with two planes, 191 without).
+      TilePlanes pl{ctx->kv32, (size_t)ctx->ing * ctx->NL * 2 * ctx->NKV * 128, 1};
       DFL_TRY(tgemm(ctx, P_INGEST_FC, WT_F16, TG_F32, ctx->w_fc_pk, H, K, ctx->xf, rows,
-                    tile_f32(ctx->fc32, H), st));
+                    tile_f32(ctx->fc32, H), st, nullptr, &pl));
       {
         ProfScope ps(ctx, P_INGEST_FC, 0, st);
-        launch_fc_norm_rows(ctx->fc32, rows, H, ctx->hidden_norm, ctx->cfg.rms_eps, ctx->xn, st);
+        launch_fc_norm_rows(pl.splits > 1 ? ctx->kv32 : ctx->fc32, pl.splits, rows, H, ctx->hidden_norm, ctx->cfg.rms_eps, ctx->xn, st);
       }
       DFL_TRY(ingest_kv_rows(ctx, ctx->xn, rows, r0, st));
     }

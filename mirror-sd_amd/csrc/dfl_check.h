@@ -161,24 +161,26 @@ inline const char* check_tile_args(int wt, int epi, const TileArgs& a, const Til
     default:
       return "unknown epilogue";
   }
-  if (p.mtw < 1 || p.mtw > 2 || (p.rbw != 1 && p.rbw != 2 && p.rbw != 4) || p.wn < 1 ||
-      p.wn > 2 || (p.kc != 32 && p.kc != 64))
+  auto pow2_to_4 = [](int v) { return v == 1 || v == 2 || v == 4; };
+  if ((p.wm != 2 && p.wm != 4) || !pow2_to_4(p.mtw) || !pow2_to_4(p.rbw) || !pow2_to_4(p.wn) ||
+      (p.kc != 32 && p.kc != 64))
     return "unknown tile shape";
+  const int tile_rows = 32 * p.wm * p.mtw;
   if (a.M < 1 || a.N < 1 || a.K < 64 || a.K % 64 || a.K % p.kc)
     return "M, N >= 1 and K a positive multiple of 64 and of the stage's k";
   if (a.N % (32 * p.rbw * p.wn)) return "N is not a multiple of the tile's columns";
   if (a.Y && a.ldy < a.N) return "output row shorter than N";
-  if (p.tiles_n != a.N / (32 * p.rbw * p.wn) || (long long)p.tiles_m * 128 * p.mtw < a.M ||
-      (long long)p.tiles_m * 128 * p.mtw >= (long long)a.M + 128 * p.mtw)
+  if (p.tiles_n != a.N / (32 * p.rbw * p.wn) || (long long)p.tiles_m * tile_rows < a.M ||
+      (long long)p.tiles_m * tile_rows >= (long long)a.M + tile_rows)
     return "tile counts do not cover the product";
   if (p.splits < 1 || p.splits > a.K / 64) return "split-K factor outside [1, K/64]";
   if (p.splits > 1 && epi != TG_F32) return "split-K writes F32 planes only";
   if (p.tail_shape >= 0) {
     if (p.tail_shape >= kNumTileShapes || p.splits != 1) return "re-tiled tail: unknown shape";
     const TileShape& u = kTileShapes[p.tail_shape];
-    if (u.wt != wt || a.K % u.kc || (128 * p.mtw) % (128 * u.mtw) ||
+    if (u.wt != wt || a.K % u.kc || tile_rows % (32 * u.wm * u.mtw) ||
         (32 * p.rbw * p.wn) % (32 * u.rbw * u.wn) || (epi == TG_SWIGLU && u.rbw % 2) ||
-        tile_nacc(u.mtw, u.rbw) != tile_nacc(p.mtw, p.rbw))
+        tile_chains(wt, u.mtw, u.rbw) != tile_chains(wt, p.mtw, p.rbw))
       return "re-tiled tail: the shape does not divide the plan's tiles";
     if (p.head_tiles < 1 || p.head_tiles >= p.tiles_m * p.tiles_n)
       return "re-tiled tail: needs head tiles and a tail";

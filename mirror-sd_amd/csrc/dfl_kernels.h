@@ -143,9 +143,10 @@ struct TileArgs {
   uint32_t samp_seed;
 };
 struct TilePlan {
-  int mtw = 0;              // m-tiles per wave: 1 (128-row workgroup tile) or 2 (256 rows)
+  int wm = 4;               // wave rows: 2 or 4
+  int mtw = 0;              // m-tiles (32 rows) per wave: 1, 2 or 4
   int rbw = 0;              // weight row-blocks (32 columns) per wave: 1, 2 or 4
-  int wn = 0;               // wave columns: 1 (4 waves) or 2 (8 waves)
+  int wn = 0;               // wave columns: 1, 2 or 4
   int kc = 0;               // k per LDS stage: 32 or 64
   int tiles_m = 0, tiles_n = 0;
   int splits = 1;           // split-K factor (F32 planes, then launch_tile_reduce)
@@ -196,8 +197,9 @@ struct FeatPtrs {
   long long ld;
 };
 void launch_concat_feats(const FeatPtrs& f, int rows, int H, half_t* out, hipStream_t st);
-// hidden_norm of the fp32 fc rows (rounded to fp16 first) into fragment-layout tiles xn.
-void launch_fc_norm_rows(const float* fc32, int rows, int H, const half_t* g, float eps,
+// hidden_norm of the fp32 fc rows (the sum of `planes` planes [rows][H], rounded to fp16 first)
+// into fragment-layout tiles xn.
+void launch_fc_norm_rows(const float* fc32, int planes, int rows, int H, const half_t* g, float eps,
                          half_t* xn, hipStream_t st);
 // Stream-K ingest inputs: concat_j(f_j) rows (f.n features of H columns, H % 8 == 0) into
 // activation fragment layout tiles [ceil(rows/32)][32][f.n*H], padding rows zero.

@@ -230,39 +230,80 @@ void launch_feats_to_afl(const FeatPtrs& f, int rows, int H, half_t* afl, hipStr
 
 // hidden_norm(fc(.)) for the ingest: fc32 [rows][H] fp32 GEMM rows, rounded to fp16 (the
 // Linear output), then RMSNorm (fp16(fp16(x * r) * g)) into fragment-layout tiles xn
-// [ceil(rows/32)][32][H] (the K|V tile GEMM's input).
-__global__ __launch_bounds__(ROW_THREADS) void fc_norm_rows_kernel(const float* __restrict__ fc32,
-                                                                   int H, const half_t* __restrict__ g,
-                                                                   float eps,
-                                                                   half_t* __restrict__ xn) {
-  __shared__ float red[16];
-  const int r = blockIdx.x;
+// [ceil(rows/32)][32][H] (the K|V tile GEMM's input).  HBM-bound (6 bytes a value): a wave
+// holds its row in registers, 8 columns a lane and step, so the row sum needs no barrier and
+// each fragment entry is one 16-byte store; the workgroup's eight consecutive rows fill the
+// 128-byte lines of the layout together.
+constexpr int FN_ROWS = 8;
+template <int NI>   // H <= 512 * NI
+__global__ __launch_bounds__(64 * FN_ROWS) void fc_norm_rows_kernel(
+    const float* __restrict__ fc32, int planes, int rows, int H, const half_t* __restrict__ g,
+    float eps, half_t* __restrict__ xn) {
+  const int lane = threadIdx.x & 63;
+  const int r = blockIdx.x * FN_ROWS + (threadIdx.x >> 6);
+  if (r >= rows) return;
   const float* src = fc32 + (size_t)r * H;
-  float v[ROW_MAXV];
-  float ss = 0.f;
+  floatx4 a[NI][2];
 #pragma unroll
-  for (int i = 0; i < ROW_MAXV; ++i) {
-    const int k = threadIdx.x + i * ROW_THREADS;
-    v[i] = 0.f;
+  for (int i = 0; i < NI; ++i) {
+    const int k = 8 * (lane + 64 * i);
+    a[i][0] = a[i][1] = (floatx4){0.f, 0.f, 0.f, 0.f};
     if (k < H) {
-      v[i] = h2f(f2h(src[k]));
-      ss += v[i] * v[i];
+      a[i][0] = *reinterpret_cast<const floatx4*>(src + k);
+      a[i][1] = *reinterpret_cast<const floatx4*>(src + k + 4);
     }
   }
-  ss = block_sum(ss, red);
+  for (int p = 1; p < planes; ++p) {
+    src += (size_t)rows * H;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int k = 8 * (lane + 64 * i);
+      if (k < H) {
+        a[i][0] += *reinterpret_cast<const floatx4*>(src + k);
+        a[i][1] += *reinterpret_cast<const floatx4*>(src + k + 4);
+      }
+    }
+  }
+  // row sum of squares: 512 partials (column mod 512; lane l's element j is number 8 l + j),
+  // summed in a fixed tree per 64 of them (across number bits 5 .. 0), the eight sums in order
+  half8_t v[NI];
+  float t[8] = {};
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[i][j] = f2h(a[i][j >> 2][j & 3]);
+      t[j] += h2f(v[i][j]) * h2f(v[i][j]);
+    }
+#pragma unroll
+  for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) t[j] += __shfl_xor(t[j], o, 64);
+  const float part = ((t[0] + t[4]) + (t[2] + t[6])) + ((t[1] + t[5]) + (t[3] + t[7]));
+  float ss = 0.f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w)
+    ss += __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(part), 8 * w));
   const float rr = 1.0f / sqrtf(ss / (float)H + eps);
 #pragma unroll
-  for (int i = 0; i < ROW_MAXV; ++i) {
-    const int k = threadIdx.x + i * ROW_THREADS;
-    if (k < H) xn[afl_index(r, k, H)] = rms_out(v[i], rr, g[k]);
+  for (int i = 0; i < NI; ++i) {
+    const int k = 8 * (lane + 64 * i);
+    if (k >= H) break;
+    const half8_t gv = *reinterpret_cast<const half8_t*>(g + k);
+    half8_t o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = rms_out_once(h2f(v[i][j]), rr, gv[j]);
+    *reinterpret_cast<half8_t*>(xn + afl_index(r, k, H)) = o;
   }
 }
 
-void launch_fc_norm_rows(const float* fc32, int rows, int H, const half_t* g, float eps,
+void launch_fc_norm_rows(const float* fc32, int planes, int rows, int H, const half_t* g, float eps,
                          half_t* xn, hipStream_t st) {
   if (rows <= 0) return;
-  hipLaunchKernelGGL(fc_norm_rows_kernel, dim3(rows), dim3(ROW_THREADS), 0, st, fc32, H, g, eps,
-                     xn);
+  // (hidden sizes up to 8192; the smaller instantiation holds half the registers)
+  auto* kernel = H <= 5120 ? fc_norm_rows_kernel<10> : fc_norm_rows_kernel<16>;
+  hipLaunchKernelGGL(kernel, dim3((rows + FN_ROWS - 1) / FN_ROWS), dim3(64 * FN_ROWS), 0, st, fc32,
+                     planes, rows, H, g, eps, xn);
 }
 
 void launch_afl_to_rows(const half_t* x, int M, int N, half_t* h, hipStream_t st) {

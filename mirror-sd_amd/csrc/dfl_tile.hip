@@ -11,11 +11,11 @@
 //
 // At M = 256 an int8 weight byte feeds 512 flop, above the MI355X ridge (~312 flop/B), so
 // these shapes are MFMA-bound rather than HBM-bound; what bounds them in practice is the
-// global -> LDS copy rate (12.5-20.5 B per cycle and CU, 8-13 TB/s over the chip, set by
-// how fast the issuing waves issue copies), so the larger the workgroup tile, the fewer
-// bytes per flop.  A workgroup of 4 * WN compute waves (WN = 1 or 2 wave columns; plus
-// four loader waves that issue every copy when WN = 1) computes a BM x BN output tile:
-// BM = 128 * MTW rows (wave row wm owns m-tiles
+// global -> LDS copy rate and the stage's chain of copy, barrier, fragment reads and MFMAs
+// (12-27 B per cycle and CU copied), so the larger the workgroup tile, the fewer bytes per
+// flop.  A workgroup of WM x WN compute waves (plus four loader waves that issue every copy
+// when that is 4 waves) computes a BM x BN output tile:
+// BM = 32 * MTW * WM rows (wave row wm owns m-tiles
 // [wm*MTW, (wm+1)*MTW)), BN = 32 * RBW * WN columns (wave column wn owns row-blocks
 // [wn*RBW, (wn+1)*RBW)).  K is walked in stages of KC (32 or 64): each stage's X records
 // (BM/32 tiles x KC/16 KiB, contiguous per tile) and weight blocks (contiguous per
@@ -55,12 +55,12 @@ DFL_DEV void tile_coords(const TileArgs& a, int tile, int& tm, int& tn) {
   tn = tig / gm;
 }
 
-template <int WT, int MTW, int RBW, int WN, int KC>
+template <int WT, int WM, int MTW, int RBW, int WN, int KC>
 struct TgShape {
-  static constexpr int NW = TG_WM * WN;                      // compute waves
-  static constexpr bool LOADER = tile_loader(WN);            // + loader waves
-  static constexpr int NLOAD = tile_loaders(WN);
-  static constexpr int MT = TG_WM * MTW;                     // m-tiles per workgroup
+  static constexpr int NW = WM * WN;                      // compute waves
+  static constexpr int NLOAD = tile_loaders(WM, WN);   // + loader waves
+  static constexpr bool LOADER = NLOAD > 0;
+  static constexpr int MT = WM * MTW;                     // m-tiles per workgroup
   static constexpr int RB = RBW * WN;                        // row-blocks per workgroup
   static constexpr int KBS = KC / 32;                        // k-blocks of 32 per stage
   static constexpr int XREC = 2 * KBS;                       // X records per tile and stage
@@ -71,14 +71,14 @@ struct TgShape {
   static constexpr int IPS = STAGE / 1024;                   // copies per stage
   // copies per issuing wave (at least)
   static constexpr int PER_WAVE_MIN = LOADER ? IPS / NLOAD : IPS / NW;
-  static constexpr int STAGES = tile_stages(WT, MTW, RBW, WN, KC);
+  static constexpr int STAGES = tile_stages(WT, WM, MTW, RBW, WN, KC);
   static constexpr int LDS = STAGES * STAGE;
-  static_assert(STAGE == tile_stage_bytes(WT, MTW, RBW, WN, KC), "stage size");
+  static_assert(STAGE == tile_stage_bytes(WT, WM, MTW, RBW, WN, KC), "stage size");
   static_assert((STAGES - 3) * (LOADER ? (IPS + NLOAD - 1) / NLOAD : (IPS + NW - 1) / NW) < 64 &&
                     STAGES >= 3,
                 "vmcnt range");
   static_assert(LDS <= TG_LDS_BUDGET, "LDS budget");
-  static constexpr int NACC = tile_nacc(MTW, RBW);           // independent MFMA chains
+  static constexpr int NACC = tile_chains(WT, MTW, RBW);
 };
 
 // s_waitcnt vmcnt(N) (gfx9 encoding: vmcnt in bits 3:0 and 15:14; expcnt and lgkmcnt
@@ -194,8 +194,7 @@ DFL_DEV void tg_mfma(const TgFrag<WT, MTW, RBW>& f, floatx16 (&acc)[RBW][MTW][NA
     static_for<0, 2>([&](auto qq) {
       static_for<0, RBW>([&](auto r) {
         static_for<0, MTW>([&](auto t) {
-          constexpr int c = NACC == 1 ? 0 : (int)qq;
-          acc[r][t][c] = mfma32x32x16(f.x[qq][t][0], as_half8(f.w[qq][r]), acc[r][t][c]);
+          acc[r][t][0] = mfma32x32x16(f.x[qq][t][0], as_half8(f.w[qq][r]), acc[r][t][0]);
         });
       });
     });
@@ -207,14 +206,14 @@ DFL_DEV void tg_mfma(const TgFrag<WT, MTW, RBW>& f, floatx16 (&acc)[RBW][MTW][NA
 // MFMAs before B(t)) before the copies of stage t + STAGES - 1 that refill its buffer,
 // issued right after B(t).  B(-1) precedes the first read.  Every wave passes B(-1) ..
 // B(nst - 2).
-template <int WT, int EPI, int MTW, int RBW, int WN, int KC>
-__global__ __launch_bounds__(64 * (TG_WM * WN + tile_loaders(WN))) void tile_gemm_kernel(
+template <int WT, int EPI, int WM, int MTW, int RBW, int WN, int KC>
+__global__ __launch_bounds__(64 * (WM * WN + tile_loaders(WM, WN))) void tile_gemm_kernel(
     TileArgs a) {
-  using S = TgShape<WT, MTW, RBW, WN, KC>;
+  using S = TgShape<WT, WM, MTW, RBW, WN, KC>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char tg_lds[];
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
-  const int wm = wv % TG_WM, wn = wv / TG_WM;
+  const int wm = wv % WM, wn = wv / WM;
 
   // XCD-aware tile order: consecutive workgroups go to different XCDs, so tile t is run by
   // workgroup b with t = (b % 8) * (G / 8) + b / 8; neighbouring tiles (sharing X or W)
@@ -476,17 +475,17 @@ __global__ __launch_bounds__(64 * (TG_WM * WN + tile_loaders(WN))) void tile_gem
   }
 }
 
-template <int WT, int EPI, int MTW, int RBW, int WN, int KC>
+template <int WT, int EPI, int WM, int MTW, int RBW, int WN, int KC>
 void launch_tile(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  using S = TgShape<WT, MTW, RBW, WN, KC>;
+  using S = TgShape<WT, WM, MTW, RBW, WN, KC>;
   const int nsub = a.pmt ? (a.pmt / S::MT) * (a.prb / S::RB) : 1;
   const dim3 grid((a.ntiles ? a.ntiles * nsub : a.tiles_m * a.tiles_n) * a.splits),
       block(64 * (S::NW + S::NLOAD));
   if (e0 || e1)
-    hipExtLaunchKernelGGL((tile_gemm_kernel<WT, EPI, MTW, RBW, WN, KC>), grid, block, S::LDS, st,
+    hipExtLaunchKernelGGL((tile_gemm_kernel<WT, EPI, WM, MTW, RBW, WN, KC>), grid, block, S::LDS, st,
                           e0, e1, 0, a);
   else
-    hipLaunchKernelGGL((tile_gemm_kernel<WT, EPI, MTW, RBW, WN, KC>), grid, block, S::LDS, st, a);
+    hipLaunchKernelGGL((tile_gemm_kernel<WT, EPI, WM, MTW, RBW, WN, KC>), grid, block, S::LDS, st, a);
 }
 
 // The epilogues each weight type has: int8 F32 / RESID / SWIGLU (gate|up pairs), fp16 F32 /
@@ -497,25 +496,25 @@ bool launch_shape_i(int wt, int epi, const TileArgs& a, const TilePlan& p, hipSt
   if constexpr (I < kNumTileShapes) {
     constexpr TileShape s = kTileShapes[I];
     if (wt == s.wt && (shape >= 0 ? shape == I
-                                  : (!s.tail && p.mtw == s.mtw && p.rbw == s.rbw &&
+                                  : (!s.tail && p.wm == s.wm && p.mtw == s.mtw && p.rbw == s.rbw &&
                                      p.wn == s.wn && p.kc == s.kc))) {
       if (epi == TG_F32) {
-        launch_tile<s.wt, TG_F32, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
+        launch_tile<s.wt, TG_F32, s.wm, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
         return true;
       }
       if constexpr (s.wt == WT_INT8) {
         if (epi == TG_RESID) {
-          launch_tile<s.wt, TG_RESID, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
+          launch_tile<s.wt, TG_RESID, s.wm, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
           return true;
         }
         if constexpr (s.rbw % 2 == 0)
           if (epi == TG_SWIGLU) {
-            launch_tile<s.wt, TG_SWIGLU, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
+            launch_tile<s.wt, TG_SWIGLU, s.wm, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
             return true;
           }
       } else {
         if (epi == TG_ARGMAX) {
-          launch_tile<s.wt, TG_ARGMAX, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
+          launch_tile<s.wt, TG_ARGMAX, s.wm, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);
           return true;
         }
       }
@@ -587,7 +586,7 @@ bool launch_tile_gemm(int wt, int epi, const TileArgs& a0, const TilePlan& p, hi
   if (!launch_shape_i<0>(wt, epi, a, p, st, ev_start, nullptr)) return false;
   a.tile0 = p.head_tiles;
   a.ntiles = p.tiles_m * p.tiles_n - p.head_tiles;
-  a.pmt = TG_WM * p.mtw;
+  a.pmt = p.wm * p.mtw;
   a.prb = p.rbw * p.wn;
   return launch_shape_i<0>(wt, epi, a, p, st, nullptr, ev_stop, p.tail_shape);
 }
