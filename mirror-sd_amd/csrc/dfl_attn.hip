@@ -41,6 +41,8 @@ constexpr int AT_STAGE_BLOCKS = 5;              // 32-key blocks per LDS stage
 constexpr int AT_KBLK = 32 * 256;               // K rows of one key block (bytes)
 constexpr int AT_VBLK = 128 * 64;               // Vt rows of one key block (bytes)
 constexpr int AT_STAGE_BYTES = AT_STAGE_BLOCKS * (AT_KBLK + AT_VBLK);
+constexpr int AT_RING = 5;                      // key blocks of the ring (80 KiB)
+constexpr int AT_RING_BYTES = AT_RING * (AT_KBLK + AT_VBLK);
 constexpr int AT_PART_BYTES = (64 * 64 + 2 * 64) * 4;   // one wave's O accumulators + (m, l)
 constexpr float AT_RESCALE = 8.f;               // log2 slack of the lazy reference max
 
@@ -51,22 +53,48 @@ DFL_DEV int vswz(int d) { return ((d >> 1) & 3) ^ ((d >> 3) & 1); }
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
+// Waits until at most N of this wave's vector memory loads are outstanding.
+template <int N>
+DFL_DEV void wait_loads() {
+  static_assert(N >= 0 && N < 16, "vmcnt bits 3:0");
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(N | (7 << 4) | (15 << 8));
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+// Barrier without the full wait of __syncthreads (loads of later blocks stay in flight); this
+// wave's LDS reads have been consumed by products before it.
+DFL_DEV void block_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 }  // namespace
 
 // PIPE (one sequence, chunks of several stages, one workgroup of <= 5 waves per CU): two
 // stage buffers (160 KiB), the next stage's loads in flight while this one computes.
+// RING (several sequences, two workgroups of 4 waves per CU, one wave per query tile): the key
+// blocks go through a ring of 5 (80 KiB), four of them in flight while one computes, with one
+// barrier a block.  With the single buffer a workgroup had no load in flight while it computed:
+// eight sequences of 40122 keys, 32 query heads of 32 rows, 57.5 -> 50.5 us (165 MB of K and V).
 // MAXW: the most waves a launch of the instantiation has.  The kernel needs about 190
 // VGPRs, so a CU holds 8 of its waves (2 per SIMD): MAXW <= 8 gives every instantiation
 // that budget (a 12-wave bound held it to 168 and spilled 21 VGPRs), and the launcher keeps
 // a workgroup's waves within 8, or 4 where two workgroups share a CU.  The two-buffer kernel
 // with 5 query tiles runs on 8 waves (SPLIT below: 32K keys 1034 vs 1050-1056 us per
 // block).
-template <bool PIPE, int MAXW>
-__global__ __launch_bounds__(64 * MAXW) void block_attn_kernel(AttnArgs a) {
+template <bool PIPE, int MAXW, bool RING = false>
+__global__ __launch_bounds__(64 * MAXW, RING ? 2 : 1) void block_attn_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int g = blockIdx.y;
   const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  int wv = threadIdx.x >> 6;
+  if constexpr (RING) wv = __builtin_amdgcn_readfirstlane(wv);
+  const int nw = blockDim.x >> 6;
   // SPLIT: the two-buffer kernel with 5 query tiles on 8 waves -- waves 0-3 take tiles 0-3
   // whole, waves 4-7 the key blocks of tile 4 round-robin (at most 7 of a stage's 25
   // tile-blocks per SIMD instead of 10); tile 4's four states merge in LDS at the end
@@ -112,163 +140,195 @@ __global__ __launch_bounds__(64 * MAXW) void block_attn_kernel(AttnArgs a) {
 
   // 16 segments per key block: 8 for K (4 key rows each), 8 for Vt (16 d rows each).
   // Keys past L are clamped to valid addresses; they are masked (K) or meet p = 0 (V).
+  // segment s of the key block at k0 to the block's K and Vt areas
+  auto issue_seg = [&](int k0, int s, unsigned char* kb, unsigned char* vb) {
+    const half_t* src;
+    unsigned char* dst;
+    if (s < 8) {
+      const int r = 4 * s + (lane >> 4);                        // key row in the block
+      const int cc = (lane & 15) ^ kswz(r);
+      const int key = min(k0 + r, sq.L - 1);
+      src = kg + (size_t)key * 128 + cc * 8;
+      dst = kb + s * 1024;
+    } else {
+      const int d = 16 * (s - 8) + (lane >> 2);
+      const int cc = (lane & 3) ^ vswz(d);
+      src = vg + (size_t)d * a.cap + min(k0 + 8 * cc, vlast);
+      dst = vb + (s - 8) * 1024;
+    }
+    __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr_t)dst, 16, 0, 0);
+  };
   auto issue_stage = [&](int k0, unsigned char* buf) {
     const int nblk = min(AT_STAGE_BLOCKS, (k_end - k0 + 31) >> 5);
     for (int sgi = wv; sgi < 16 * nblk; sgi += nw) {
-      const int j = sgi >> 4, s = sgi & 15;
-      const half_t* src;
-      unsigned char* dst;
-      if (s < 8) {
-        const int r = 4 * s + (lane >> 4);                        // key row in the block
-        const int cc = (lane & 15) ^ kswz(r);
-        const int key = min(k0 + 32 * j + r, sq.L - 1);
-        src = kg + (size_t)key * 128 + cc * 8;
-        dst = buf + j * AT_KBLK + s * 1024;
-      } else {
-        const int d = 16 * (s - 8) + (lane >> 2);
-        const int cc = (lane & 3) ^ vswz(d);
-        src = vg + (size_t)d * a.cap + min(k0 + 32 * j + 8 * cc, vlast);
-        dst = buf + AT_STAGE_BLOCKS * AT_KBLK + j * AT_VBLK + (s - 8) * 1024;
-      }
-      __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr_t)dst, 16, 0, 0);
+      const int j = sgi >> 4;
+      issue_seg(k0 + 32 * j, sgi & 15, buf + j * AT_KBLK,
+                buf + AT_STAGE_BLOCKS * AT_KBLK + j * AT_VBLK);
     }
   };
-  // One buffer: issue a stage, wait, compute, repeat.  PIPE: the buffers alternate, and the
-  // next stage is issued into the other one before this one computes.
-  int k0 = k_begin, p = 0;
-  issue_stage(k0, lds);
-#pragma unroll
-  for (int st = 0; st < 8; ++st) qf[st] = as_half8(qp[st]);   // overlaps the first stage
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  for (;;) {
-    const int nblk = min(AT_STAGE_BLOCKS, (k_end - k0 + 31) >> 5);
-    const int kn = k0 + 32 * AT_STAGE_BLOCKS;
-    const unsigned char* buf = lds + (PIPE ? p * AT_STAGE_BYTES : 0);
-    if (PIPE && kn < k_end) issue_stage(kn, lds + (p ^ 1) * AT_STAGE_BYTES);
-
-    for (int j = kwi; j < nblk; j += KW) {
-      const unsigned char* kb_lds = buf + j * AT_KBLK + koff * 256;
-      const unsigned char* vb_lds = buf + AT_STAGE_BLOCKS * AT_KBLK + j * AT_VBLK;
-      floatx16 s = {};
-      u32x4 vf[4][2];
-      if constexpr (PIPE) {
-        // all eight K fragment reads in flight before the first product, and the V
-        // fragments read while the softmax runs (the two-buffer kernel has the registers)
-        u32x4 kf[8];
-        static_for<0, 8>([&](auto st) {
-          kf[st] = *reinterpret_cast<const u32x4*>(kb_lds + (((8 * gg + st) ^ kxor) << 4));
-        });
-        __builtin_amdgcn_sched_barrier(0);
-        static_for<0, 8>([&](auto st) { s = mfma32x32x16(as_half8(kf[st]), qf[st], s); });
-        static_for<0, 4>([&](auto dt) {
-          const unsigned char* vr = vb_lds + (dt * 32 + vrow) * 64;
-          const int vx = vswz(dt * 32 + vrow);
-          vf[dt][0] = *reinterpret_cast<const u32x4*>(vr + ((gg ^ vx) << 4));
-          vf[dt][1] = *reinterpret_cast<const u32x4*>(vr + (((gg + 2) ^ vx) << 4));
-        });
-        __builtin_amdgcn_sched_barrier(0);
-      } else {
-        static_for<0, 8>([&](auto st) {
-          const u32x4 kf =
-              *reinterpret_cast<const u32x4*>(kb_lds + (((8 * gg + st) ^ kxor) << 4));
-          s = mfma32x32x16(as_half8(kf), qf[st], s);
-        });
-      }
-      // Accumulator r holds key kbase + (r < 8 ? 8*gg + r : 16 + 8*gg + r - 8).
-      const int kbase = k0 + 32 * j;
-      float psum = 0.f;
-      half8_t p1, p2;
-      // rescale o and lrun when the block's max exceeds the lazy reference by > AT_RESCALE
-      auto update_ref = [&](float bmax) {
-        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-        if (!__all(bmax <= mrun + AT_RESCALE)) {
-          const float mnew = bmax > mrun + AT_RESCALE ? bmax : mrun;
-          const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);
-          lrun *= alpha;
-          static_for<0, 4>([&](auto dt) { o[dt] *= alpha; });
-          mrun = mnew;
-        }
-      };
-      if (sq.ring_W == 0 && kbase + 32 <= k_end) {
-        // every key valid: max(s * c) = max(s) * c (c > 0, rounding is monotonic), and mrun
-        // is finite after update_ref, so p = 2^(s * c - mrun) needs no mask; p in fp16 two
-        // per v_cvt_pk, the row sum of the fp16 p two per v_dot2 (half the VALU work of the
-        // masked path, which bounds the compute of long chunks: 32K keys 1053 vs 1085 us
-        // per block)
-        float smax = s[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) smax = fmaxf(smax, s[r]);
-        update_ref(smax * a.scale_log2);
-        const half2_t one2 = {(half_t)1.0f, (half_t)1.0f};
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const half2_t ph = __builtin_convertvector(
-              ((floatx2){__builtin_amdgcn_exp2f(__builtin_fmaf(s[r], a.scale_log2, -mrun)),
-                         __builtin_amdgcn_exp2f(__builtin_fmaf(s[r + 1], a.scale_log2, -mrun))}),
-              half2_t);
-          psum = __builtin_amdgcn_fdot2(ph, one2, psum, false);
-          if (r < 8) { p1[r] = ph.x; p1[r + 1] = ph.y; } else { p2[r - 8] = ph.x; p2[r - 7] = ph.y; }
-        }
-      } else {
-        float v[16];
-        if (sq.ring_W > 0) {   // sink + window cache: only the valid ring rows count
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int kr = kbase + (r < 8 ? 8 * gg + r : 16 + 8 * gg + (r - 8));
-            bool ok = kr < k_end;
-            if (kr < sq.ring_S) {
-              ok = ok && kr < sq.sink_len;
-            } else {
-              const int back = (sq.ring_j - 1 - (kr - sq.ring_S)) % sq.ring_W;
-              ok = ok && (back < 0 ? back + sq.ring_W : back) < sq.ring_len;
-            }
-            v[r] = ok ? s[r] * a.scale_log2 : -INFINITY;
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int kr = kbase + (r < 8 ? 8 * gg + r : 16 + 8 * gg + (r - 8));
-            v[r] = kr < k_end ? s[r] * a.scale_log2 : -INFINITY;
-          }
-        }
-        float bmax = v[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) bmax = fmaxf(bmax, v[r]);
-        update_ref(bmax);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          // masked keys contribute 0 (also when every key so far was masked, mrun = -inf)
-          const half_t ph = v[r] == -INFINITY ? (half_t)0.0f : f2h(__builtin_amdgcn_exp2f(v[r] - mrun));
-          psum += h2f(ph);
-          if (r < 8) p1[r] = ph; else p2[r - 8] = ph;
-        }
-      }
-      lrun += psum + __shfl_xor(psum, 32, 64);
+  // one 32-key block: kb_lds is this lane's K row, vb_lds the block's Vt area, kbase its key 0
+  auto key_block = [&](const unsigned char* kb_lds, const unsigned char* vb_lds, int kbase)
+      __attribute__((always_inline)) {
+    floatx16 s = {};
+    u32x4 vf[4][2];
+    if constexpr (PIPE || RING) {
+      // all eight K fragment reads in flight before the first product, and the V
+      // fragments read while the softmax runs (the two-buffer kernel has the registers)
+      u32x4 kf[8];
+      static_for<0, 8>([&](auto st) {
+        kf[st] = *reinterpret_cast<const u32x4*>(kb_lds + (((8 * gg + st) ^ kxor) << 4));
+      });
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<0, 8>([&](auto st) { s = mfma32x32x16(as_half8(kf[st]), qf[st], s); });
       static_for<0, 4>([&](auto dt) {
-        u32x4 v1, v2;
-        if constexpr (PIPE) {
-          v1 = vf[dt][0];
-          v2 = vf[dt][1];
-        } else {
-          const unsigned char* vr = vb_lds + (dt * 32 + vrow) * 64;
-          const int vx = vswz(dt * 32 + vrow);
-          v1 = *reinterpret_cast<const u32x4*>(vr + ((gg ^ vx) << 4));
-          v2 = *reinterpret_cast<const u32x4*>(vr + (((gg + 2) ^ vx) << 4));
-        }
-        o[dt] = mfma32x32x16(as_half8(v1), p1, o[dt]);
-        o[dt] = mfma32x32x16(as_half8(v2), p2, o[dt]);
+        const unsigned char* vr = vb_lds + (dt * 32 + vrow) * 64;
+        const int vx = vswz(dt * 32 + vrow);
+        vf[dt][0] = *reinterpret_cast<const u32x4*>(vr + ((gg ^ vx) << 4));
+        vf[dt][1] = *reinterpret_cast<const u32x4*>(vr + (((gg + 2) ^ vx) << 4));
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      static_for<0, 8>([&](auto st) {
+        const u32x4 kf =
+            *reinterpret_cast<const u32x4*>(kb_lds + (((8 * gg + st) ^ kxor) << 4));
+        s = mfma32x32x16(as_half8(kf), qf[st], s);
       });
     }
-    if (kn >= k_end) break;
-    if (!PIPE) {
-      __syncthreads();   // every wave is done with the single buffer
-      issue_stage(kn, lds);
+    // Accumulator r holds key kbase + (r < 8 ? 8*gg + r : 16 + 8*gg + r - 8).
+    float psum = 0.f;
+    half8_t p1, p2;
+    // rescale o and lrun when the block's max exceeds the lazy reference by > AT_RESCALE
+    auto update_ref = [&](float bmax) {
+      bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+      if (!__all(bmax <= mrun + AT_RESCALE)) {
+        const float mnew = bmax > mrun + AT_RESCALE ? bmax : mrun;
+        const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);
+        lrun *= alpha;
+        static_for<0, 4>([&](auto dt) { o[dt] *= alpha; });
+        mrun = mnew;
+      }
+    };
+    if (sq.ring_W == 0 && kbase + 32 <= k_end) {
+      // every key valid: max(s * c) = max(s) * c (c > 0, rounding is monotonic), and mrun
+      // is finite after update_ref, so p = 2^(s * c - mrun) needs no mask; p in fp16 two
+      // per v_cvt_pk, the row sum of the fp16 p two per v_dot2 (half the VALU work of the
+      // masked path, which bounds the compute of long chunks: 32K keys 1053 vs 1085 us
+      // per block)
+      float smax = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) smax = fmaxf(smax, s[r]);
+      update_ref(smax * a.scale_log2);
+      const half2_t one2 = {(half_t)1.0f, (half_t)1.0f};
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        const half2_t ph = __builtin_convertvector(
+            ((floatx2){__builtin_amdgcn_exp2f(__builtin_fmaf(s[r], a.scale_log2, -mrun)),
+                       __builtin_amdgcn_exp2f(__builtin_fmaf(s[r + 1], a.scale_log2, -mrun))}),
+            half2_t);
+        psum = __builtin_amdgcn_fdot2(ph, one2, psum, false);
+        if (r < 8) { p1[r] = ph.x; p1[r + 1] = ph.y; } else { p2[r - 8] = ph.x; p2[r - 7] = ph.y; }
+      }
+    } else {
+      float v[16];
+      if (sq.ring_W > 0) {   // sink + window cache: only the valid ring rows count
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kr = kbase + (r < 8 ? 8 * gg + r : 16 + 8 * gg + (r - 8));
+          bool ok = kr < k_end;
+          if (kr < sq.ring_S) {
+            ok = ok && kr < sq.sink_len;
+          } else {
+            const int back = (sq.ring_j - 1 - (kr - sq.ring_S)) % sq.ring_W;
+            ok = ok && (back < 0 ? back + sq.ring_W : back) < sq.ring_len;
+          }
+          v[r] = ok ? s[r] * a.scale_log2 : -INFINITY;
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kr = kbase + (r < 8 ? 8 * gg + r : 16 + 8 * gg + (r - 8));
+          v[r] = kr < k_end ? s[r] * a.scale_log2 : -INFINITY;
+        }
+      }
+      float bmax = v[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) bmax = fmaxf(bmax, v[r]);
+      update_ref(bmax);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        // masked keys contribute 0 (also when every key so far was masked, mrun = -inf)
+        const half_t ph = v[r] == -INFINITY ? (half_t)0.0f : f2h(__builtin_amdgcn_exp2f(v[r] - mrun));
+        psum += h2f(ph);
+        if (r < 8) p1[r] = ph; else p2[r - 8] = ph;
+      }
     }
-    __builtin_amdgcn_s_waitcnt(0);   // this wave's loads of the next stage have landed
-    __syncthreads();                 // everyone's, and no wave reads the buffer they reuse
-    k0 = kn;
-    p ^= 1;
+    lrun += psum + __shfl_xor(psum, 32, 64);
+    static_for<0, 4>([&](auto dt) {
+      u32x4 v1, v2;
+      if constexpr (PIPE || RING) {
+        v1 = vf[dt][0];
+        v2 = vf[dt][1];
+      } else {
+        const unsigned char* vr = vb_lds + (dt * 32 + vrow) * 64;
+        const int vx = vswz(dt * 32 + vrow);
+        v1 = *reinterpret_cast<const u32x4*>(vr + ((gg ^ vx) << 4));
+        v2 = *reinterpret_cast<const u32x4*>(vr + (((gg + 2) ^ vx) << 4));
+      }
+      o[dt] = mfma32x32x16(as_half8(v1), p1, o[dt]);
+      o[dt] = mfma32x32x16(as_half8(v2), p2, o[dt]);
+    });
+  };
+  if constexpr (RING) {
+    // block j is at ring slot j % AT_RING; 4 waves: 4 segments a wave and block, so the
+    // blocks behind block j are 4 loads each in a wave's count
+    const int nblk = (k_end - k_begin + 31) >> 5;
+    auto issue_block = [&](int j) {
+      unsigned char* kb = lds + (j % AT_RING) * (AT_KBLK + AT_VBLK);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) issue_seg(k_begin + 32 * j, wv + 4 * i, kb, kb + AT_KBLK);
+    };
+    for (int st = 0; st < 8; ++st) qf[st] = as_half8(qp[st]);
+    __builtin_amdgcn_s_waitcnt(0);   // (the counts below are the ring's loads alone)
+    for (int j = 0; j < AT_RING - 1 && j < nblk; ++j) issue_block(j);
+    for (int j = 0; j < nblk; ++j) {
+      const int behind = min(AT_RING - 2, nblk - 1 - j);   // younger blocks in flight
+      if (behind == 3) wait_loads<12>();
+      else if (behind == 2) wait_loads<8>();
+      else if (behind == 1) wait_loads<4>();
+      else wait_loads<0>();
+      block_barrier();   // everyone's segments of block j; nobody reads block j - 1 any more
+      if (j + AT_RING - 1 < nblk) issue_block(j + AT_RING - 1);
+      const unsigned char* kb = lds + (j % AT_RING) * (AT_KBLK + AT_VBLK);
+      key_block(kb + koff * 256, kb + AT_KBLK, k_begin + 32 * j);
+    }
+  } else {
+    // One buffer: issue a stage, wait, compute, repeat.  PIPE: the buffers alternate, and the
+    // next stage is issued into the other one before this one computes.
+    int k0 = k_begin, p = 0;
+    issue_stage(k0, lds);
+#pragma unroll
+    for (int st = 0; st < 8; ++st) qf[st] = as_half8(qp[st]);   // overlaps the first stage
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    for (;;) {
+      const int nblk = min(AT_STAGE_BLOCKS, (k_end - k0 + 31) >> 5);
+      const int kn = k0 + 32 * AT_STAGE_BLOCKS;
+      const unsigned char* buf = lds + (PIPE ? p * AT_STAGE_BYTES : 0);
+      if (PIPE && kn < k_end) issue_stage(kn, lds + (p ^ 1) * AT_STAGE_BYTES);
+
+      for (int j = kwi; j < nblk; j += KW)
+        key_block(buf + j * AT_KBLK + koff * 256,
+                  buf + AT_STAGE_BLOCKS * AT_KBLK + j * AT_VBLK, k0 + 32 * j);
+      if (kn >= k_end) break;
+      if (!PIPE) {
+        __syncthreads();   // every wave is done with the single buffer
+        issue_stage(kn, lds);
+      }
+      __builtin_amdgcn_s_waitcnt(0);   // this wave's loads of the next stage have landed
+      __syncthreads();                 // everyone's, and no wave reads the buffer they reuse
+      k0 = kn;
+      p ^= 1;
+    }
   }
   __syncthreads();   // the stage buffers are reused by the merge
 
@@ -366,6 +426,67 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(AttnArgs a) {
   a.O[afl_index(orow, h * 128 + d, a.NH * 128)] = f2h(num / den_s);
 }
 
+// The same with half a wave per row and 16 bytes a lane and chunk (a quarter of the load
+// instructions, no barrier), in the same order of sums: 8192 rows of up to 13 chunks 9.7 us
+// against 12.9; but fewer waves to hide the loads behind, 1280 rows of 26 chunks 6.5 against 5.0.
+constexpr int MERGE_WIDE_ROWS = 8;      // rows per workgroup
+constexpr int MERGE_WIDE_MIN = 4096;    // rows from which a launch uses it
+__global__ __launch_bounds__(32 * MERGE_WIDE_ROWS) void attn_merge_wide_kernel(AttnArgs a,
+                                                                               int n_rows) {
+  __shared__ float wts[MERGE_WIDE_ROWS][64];
+  const int l = threadIdx.x & 31, wr = threadIdx.x >> 5;
+  const int rowg = blockIdx.x * MERGE_WIDE_ROWS + wr;   // s * NH * B + h * B + b
+  if (rowg >= n_rows) return;   // (its half wave; no barrier below)
+  const int per_seq = a.NH * a.B;
+  const int sidx = rowg / per_seq;
+  const size_t NB = (size_t)a.n_seq * per_seq;
+  const int nc = a.sq[sidx].n_chunks;   // <= MAX_CHUNKS = 64: chunks l and l + 32 of this lane
+  constexpr int C = 16;
+  const float* op = a.Op + (size_t)rowg * 128 + 4 * l;
+  floatx4 v[C];
+#pragma unroll
+  for (int j = 0; j < C; ++j)
+    v[j] = j < nc ? *reinterpret_cast<const floatx4*>(op + (size_t)j * NB * 128)
+                  : (floatx4){0.f, 0.f, 0.f, 0.f};
+  floatx2 q0 = {-INFINITY, 0.f}, q1 = {-INFINITY, 0.f};
+  if (l < nc) q0 = *reinterpret_cast<const floatx2*>(a.Ml + ((size_t)l * NB + rowg) * 2);
+  if (l + 32 < nc) q1 = *reinterpret_cast<const floatx2*>(a.Ml + ((size_t)(l + 32) * NB + rowg) * 2);
+  float M = fmaxf(q0.x, q1.x);
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+  const float w0 = l < nc ? exp2f(q0.x - M) : 0.f, w1 = l + 32 < nc ? exp2f(q1.x - M) : 0.f;
+  wts[wr][l] = w0;
+  wts[wr][l + 32] = w1;
+  float den = w0 * q0.y, den1 = w1 * q1.y;
+  asm volatile("" : "+v"(den1));   // both products rounded (not one of them fused)
+  den += den1;
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) den += __shfl_xor(den, o, 64);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the row's weights, one wave's own
+  floatx4 num = {0.f, 0.f, 0.f, 0.f};
+  for (int c0 = 0;;) {
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+      if (c0 + j < nc) {
+        const float w = wts[wr][c0 + j];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) num[k] = __builtin_fmaf(v[j][k], w, num[k]);
+      }
+    c0 += C;
+    if (c0 >= nc) break;
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+      if (c0 + j < nc) v[j] = *reinterpret_cast<const floatx4*>(op + (size_t)(c0 + j) * NB * 128);
+  }
+  const int hb = rowg - sidx * per_seq;
+  const int h = hb / a.B, b = hb - h * a.B;
+  const int orow = a.sq[sidx].o_row0 + b;
+  half4_t o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = f2h(num[k] / den);
+  *reinterpret_cast<half4_t*>(a.O + afl_index(orow, h * 128 + 4 * l, a.NH * 128)) = o;
+}
+
 bool launch_block_attention(const AttnArgs& a_in, hipStream_t st) {
   if (check_attn_args(a_in)) return false;
   AttnArgs a = a_in;
@@ -390,16 +511,25 @@ bool launch_block_attention(const AttnArgs& a_in, hipStream_t st) {
   const bool pipe = a.n_seq == 1 && a.sq[0].chunk > 32 * AT_STAGE_BLOCKS && a.kw == 1 &&
                     a.q_per_group <= 5 && (long long)a.chunk0[1] * a.NKV * groups <= a.n_cu &&
                     a.lds_max >= 2 * AT_STAGE_BYTES;
+  // (a wave takes every key block of its tile in order, so the sums are the single buffer's)
+  const bool ring = a.n_seq > 1 && a.kw == 1 && a.q_per_group == 4;
   const dim3 grid(a.chunk0[a.n_seq], a.NKV, groups), block(64 * a.q_per_group * a.kw);
   if (pipe && a.q_per_group == 5)
     hipLaunchKernelGGL((block_attn_kernel<true, 8>), grid, dim3(512), 2 * AT_STAGE_BYTES, st, a);
   else if (pipe)
     hipLaunchKernelGGL((block_attn_kernel<true, 5>), grid, block, 2 * AT_STAGE_BYTES, st, a);
+  else if (ring)
+    hipLaunchKernelGGL((block_attn_kernel<false, 4, true>), grid, block, AT_RING_BYTES, st, a);
   else if (a.q_per_group * a.kw <= 5)
     hipLaunchKernelGGL((block_attn_kernel<false, 5>), grid, block, lds_bytes, st, a);
   else
     hipLaunchKernelGGL((block_attn_kernel<false, 8>), grid, block, lds_bytes, st, a);
-  hipLaunchKernelGGL(attn_merge_kernel, dim3(a.n_seq * a.NH * a.B), dim3(128), 0, st, a);
+  const int rows = a.n_seq * a.NH * a.B;
+  if (rows >= MERGE_WIDE_MIN)
+    hipLaunchKernelGGL(attn_merge_wide_kernel, dim3((rows + MERGE_WIDE_ROWS - 1) / MERGE_WIDE_ROWS),
+                       dim3(32 * MERGE_WIDE_ROWS), 0, st, a, rows);
+  else
+    hipLaunchKernelGGL(attn_merge_kernel, dim3(rows), dim3(128), 0, st, a);
   return true;
 }
 
