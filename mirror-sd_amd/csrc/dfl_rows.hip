@@ -489,11 +489,14 @@ DFL_DEV void qk_rope_item(const QKRopeArgs& a, int sidx, int m, int slot, int L)
 }
 
 // Q/K part: qk_rope_item per (sequence, row, slot).
-// V part: the workgroup reads its 64 rows x 128 values row by row (coalesced), transposes
-// them through LDS and writes each Vt row d as 64 consecutive cache columns, so the
-// transposed cache layout costs no scattered 2-byte stores.
+// V part: the workgroup reads its 64 rows x 128 values (each thread two adjacent rows of four
+// columns, all its loads in flight together), transposes them through LDS and writes each Vt row
+// d as 64 consecutive cache columns, four to a store where they are consecutive and aligned, so
+// the transposed cache layout costs no scattered 2-byte stores.  Whole launch, 5 layers: 4096
+// rows (252 MB) 69 -> 65 us, 777 rows 19.7 -> 16.8, against one load in flight a thread and
+// 2-byte LDS and cache accesses.
 __global__ __launch_bounds__(256) void qk_rope_kernel(QKRopeArgs a) {
-  __shared__ half_t vt_s[128][66];   // [d][row], rows padded against bank conflicts
+  __shared__ __attribute__((aligned(16))) half_t vt_s[128][68];   // [d][row], padded
   const QkRopeGrid gr = qk_rope_grid(a);
   if ((long long)blockIdx.x >= gr.qk_blocks) {
     const long long vb = (long long)blockIdx.x - gr.qk_blocks;
@@ -502,26 +505,49 @@ __global__ __launch_bounds__(256) void qk_rope_kernel(QKRopeArgs a) {
     const int sidx = (int)(sv / gr.nv), slot = gr.v0 + (int)(sv % gr.nv);
     const RopeSeq& sq = a.sq[sidx];
     const int m0 = tile * 64;
-    for (int i = threadIdx.x; i < 64 * 32; i += 256) {
-      const int r = i >> 5, d = (i & 31) * 4;
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (m0 + r < a.M) {
+    float v[4][2][4];
+    const int d0 = (threadIdx.x & 31) * 4, r0 = 2 * (threadIdx.x >> 5);   // + 16 per step
+    static_for<0, 4>([&](auto i) {
+      static_for<0, 2>([&](auto h) {
         size_t row;
-        int c0;
-        qk_rope_src(a, sidx, m0 + r, slot, row, c0);
-        qk_rope_values<4>(a, row, c0 + d, v);
-      }
+        int c0;   // (rows past M: any valid one, never stored)
+        qk_rope_src(a, sidx, min(m0 + r0 + 16 * i + h, a.M - 1), slot, row, c0);
+        qk_rope_values<4>(a, row, c0 + d0, v[i][h]);
+      });
+    });
+    static_for<0, 4>([&](auto i) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) vt_s[d + k][r] = f2h(v[k]);
-    }
+      for (int k = 0; k < 4; ++k)
+        *reinterpret_cast<half2_t*>(&vt_s[d0 + k][r0 + 16 * i]) =
+            (half2_t){f2h(v[i][0][k]), f2h(v[i][1][k])};
+    });
     __syncthreads();
     const int gk = slot - (a.NH + a.NKV);
     half_t* vt = sq.Vt + (size_t)gk * 128 * a.cap;
-    for (int i = threadIdx.x; i < 64 * 128; i += 256) {
-      const int d = i >> 6, r = i & 63;
-      if (m0 + r >= a.M) continue;
-      const int crow = cache_slot(sq, a.M, m0 + r);
-      if (crow >= 0) vt[(size_t)d * a.cap + crow] = vt_s[d][r];
+    // this thread's four rows, in every Vt row d of its 16 d groups
+    const int r = 4 * (threadIdx.x & 15), m = m0 + r;
+    if (m >= a.M) return;
+    int crow[4];
+    bool run = m + 3 < a.M;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      crow[j] = m + j < a.M ? cache_slot(sq, a.M, m + j) : -1;
+      run = run && crow[j] == crow[0] + j;
+    }
+    run = run && crow[0] >= 0 && crow[0] % 4 == 0 && a.cap % 4 == 0 &&
+          !(reinterpret_cast<uintptr_t>(sq.Vt) & 7);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int d = (threadIdx.x >> 4) + 16 * i;
+      const half4_t h = *reinterpret_cast<const half4_t*>(&vt_s[d][r]);
+      half_t* dst = vt + (size_t)d * a.cap;
+      if (run) {
+        *reinterpret_cast<half4_t*>(dst + crow[0]) = h;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (crow[j] >= 0) dst[crow[j]] = h[j];
+      }
     }
     return;
   }
