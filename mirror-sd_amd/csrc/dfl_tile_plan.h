@@ -149,6 +149,19 @@ inline TilePlan tile_plan(int M, int N, int K, int wt, int n_cu, bool pairs = fa
   return best;
 }
 
+// Floats of the split-K planes that a product of 1 .. rows rows may be planned with (an F32 or
+// RESID product with re-tiled last rounds): the most over every row count, as neither the factor
+// nor the planes grow evenly with the rows.  A workspace of this size holds every plan, so that
+// a product's split, and with it the order of its sums, is a rule on the product alone.
+inline size_t tile_plane_floats(int rows, int N, int K, int wt, int n_cu) {
+  size_t most = 0;
+  for (int M = 1; M <= rows; ++M) {
+    const TilePlan p = tile_plan(M, N, K, wt, n_cu, false, true, true);
+    if (p.splits > 1) most = std::max(most, (size_t)p.splits * M * N);
+  }
+  return most;
+}
+
 inline size_t tile_lds_bytes(int wt, const TilePlan& p) {
   return (size_t)tile_stages(wt, p.wm, p.mtw, p.rbw, p.wn, p.kc) *
          tile_stage_bytes(wt, p.wm, p.mtw, p.rbw, p.wn, p.kc);

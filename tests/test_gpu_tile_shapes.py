@@ -97,3 +97,30 @@ def test_append_through_window(model, first, rows):
     m.make_cache(0, 0)
     assert len(keep) == slots.numel()
     _check(model, th, slots, torch.tensor(keep, device="cuda"))
+
+
+def _small(heads, kv, layers, F, **sizes):
+    from mirror_sd_amd.dflash import DFlashDraftModel
+    cfg = DFlashConfig(hidden_size=H, num_hidden_layers=layers, intermediate_size=F,
+                       num_attention_heads=heads, num_key_value_heads=kv, head_dim=128,
+                       vocab_size=512, block_size=8, target_layer_ids=[0, 1, 2, 3, 4],
+                       num_target_layers=6)
+    m = DFlashDraftModel(cfg, **sizes)
+    m.load_weights(torch_tensors(synth.make_weights_numpy(cfg, seed=11), "cuda"))
+    return m
+
+
+@pytest.mark.parametrize("rows", [65, 100, 257, 600])
+def test_rows_do_not_depend_on_the_models_size(rows):
+    """A prompt's cached rows are the same bits whatever number of context rows and layers the
+    model was made for (the fc's split over K is a rule on the product alone)."""
+    th, got = _rows(rows), []
+    for layers, ctx in ((1, rows), (1, 4096), (3, rows)):
+        m = _small(4, 4, layers, 512, max_ctx=ctx)
+        m.ingest_seq(0, th)
+        k, vt = m.cache_tensors(0)[0]
+        got.append((k[:, :rows].clone(), vt[:, :, :rows].clone()))
+        torch.cuda.synchronize()
+        m.close()
+    for k, vt in got[1:]:
+        assert torch.equal(k, got[0][0]) and torch.equal(vt, got[0][1]), rows
