@@ -400,16 +400,14 @@ int dfl_create(const dfl_config* cfg, dfl_ctx** out) {
     return r;
   }
   if (x->RM > STACK_MIN_ROWS) {
-    // split-K planes: the largest plan of the stacked qkv / o / down products over every
-    // row count up to RM
-    for (int M = 32; M <= ((x->RM + 31) / 32) * 32; M += 32)
-      for (auto nk : {std::make_pair(x->NQKV, x->H), std::make_pair(x->H, x->NH * 128),
-                      std::make_pair(x->H, x->F)}) {
-        const TilePlan p = tile_plan(std::min(M, x->RM), nk.first, nk.second, WT_INT8, x->n_cu,
-                                     false, true);
+    // split-K planes of the stacked qkv / o / down products and of a logits-only lm_head (which
+    // a small vocabulary splits), of any row count up to RM
+    struct { int N, K, wt; } split[] = {{x->NQKV, x->H, WT_INT8}, {x->H, x->NH * 128, WT_INT8},
+                                        {x->H, x->F, WT_INT8}, {x->V, x->H, WT_F16}};
+    for (const auto& s : split)
+      if (s.N > 0)
         x->tile_ws_floats =
-            std::max(x->tile_ws_floats, (size_t)p.splits * std::min(M, x->RM) * nk.first);
-      }
+            std::max(x->tile_ws_floats, tile_plane_floats(x->RM, s.N, s.K, s.wt, x->n_cu));
     if ((r = x->alloc(&x->y32, (size_t)x->RM * std::max({x->NQKV, x->H, 2 * x->F}))) ||
         (r = x->alloc(&x->tile_ws, x->tile_ws_floats))) {
       delete x;
@@ -649,9 +647,9 @@ static int tgemm(dfl_ctx* ctx, int cat, int wt, int epi, const uint4* W, int N, 
   // re-tiled last rounds for the epilogues whose outputs do not depend on the tile shape
   // (the ARGMAX keys are per wave column)
   const bool retile = epi != TG_ARGMAX;
-  TilePlan p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, split_ok, retile, chains);
-  if (p.splits > 1 && (size_t)p.splits * M * N > ws_floats)   // planes do not fit
-    p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, false, retile, chains);
+  const TilePlan p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, split_ok, retile, chains);
+  if (p.splits > 1 && (size_t)p.splits * M * N > ws_floats)   // (sized for every plan at create)
+    return fail(DFL_EINVAL, "tile GEMM: the split-K planes exceed their workspace");
   if (n_parts) *n_parts = N / (32 * p.rbw);
   TileArgs a = e;
   a.W = W;

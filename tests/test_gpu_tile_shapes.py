@@ -5,7 +5,7 @@ one through the rotation): at most 5 * 2^-11 of each row's 2-norm."""
 
 import pytest
 
-from mirror_sd_amd import synth
+from mirror_sd_amd import _lib, synth
 from mirror_sd_amd.config import DFlashConfig
 from parity_util import torch_tensors
 
@@ -124,3 +124,28 @@ def test_rows_do_not_depend_on_the_models_size(rows):
         m.close()
     for k, vt in got[1:]:
         assert torch.equal(k, got[0][0]) and torch.equal(vt, got[0][1]), rows
+
+
+@pytest.mark.parametrize("n_seq,block", [(2, 34), (2, 48)])
+def test_stacked_block_does_not_depend_on_max_seqs(n_seq, block):
+    """A stacked block's hidden states and logits are the same bits whatever number of sequences
+    the model was made for (68 rows split the down product over K 16 ways, and the lm_head of
+    512 columns where no ids are asked for).  Logits: fp32 sums of 1024 products in another
+    order, 1024 * 2^-24 of their 2-norm at most."""
+    th, got = _rows(40), []
+    ids = (torch.arange(n_seq * block, dtype=torch.int32) % 512).reshape(n_seq, block).cuda()
+    for seqs in (n_seq, 8):
+        m = _small(4, 2, 1, 3584, max_ctx=40, max_block=48, max_seqs=seqs)
+        for s in range(n_seq):
+            m.ingest_seq(s, th)
+        _, logits, hidden = m.draft_batch(ids=ids, return_logits=True, return_hidden=True)
+        alone = torch.empty_like(logits)   # without ids
+        _lib.check(m._L.dfl_draft_batch(m._ctx, n_seq, None, ids.data_ptr(), block, None, None,
+                                        alone.data_ptr(), None, _lib.stream_handle()), "logits")
+        got.append((hidden.clone(), logits.clone(), alone))
+        torch.cuda.synchronize()
+        m.close()
+    for a, b in zip(*got):
+        assert torch.equal(a, b), (n_seq, block)
+    _, logits, alone = got[0]
+    assert float((logits - alone).norm()) <= 1024 * 2.0 ** -24 * float(logits.norm())
