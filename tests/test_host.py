@@ -386,3 +386,30 @@ def test_rocprof_summary_groups_match_the_built_kernels():
                          check=True).stdout.split("\n")
     built = {n.strip() for n in out if n.strip()}
     assert set(expect) <= built, sorted(set(expect) - built)
+
+
+def test_rocprof_summary_groups_cover_a_batched_profile():
+    """Every kernel that a stacked block or a prompt-sized ingest launches falls into one group of
+    the profile summariser (a kernel in none would silently be missing from its table); the 128 x
+    128 fp16 product is not said to be a last round only."""
+    import json
+    import shutil
+    import subprocess
+    from mirror_sd_amd import rocprof_summary as rs
+    def hits(name):
+        return [g for g, rx in rs.GROUPS if re.search(rx, name) and g != "proj_gemm_w8a16"]
+    assert hits("dfl::attn_merge_kernel(dfl::AttnArgs)") == ["attention merge"]
+    assert hits("dfl::attn_merge_wide_kernel(dfl::AttnArgs, int)") == ["attention merge"]
+    fc = hits("void dfl::(anonymous namespace)::tile_gemm_kernel<1, 0, 4, 1, 4, 1, 64>(dfl::TileArgs)")
+    assert len(fc) == 1 and "few rows" in fc[0], fc
+    res = os.path.join(ROOT, "mirror-sd_amd", "_build", "kernel_resources.json")
+    if not (os.path.exists(res) and shutil.which("c++filt")):
+        pytest.skip("no build record or c++filt")
+    with open(res) as f:
+        out = subprocess.run(["c++filt"], input="\n".join(json.load(f)), capture_output=True,
+                             text=True, check=True).stdout.split("\n")
+    rx = r"tile_|attn_|rope_|afl|fc_norm_rows|embed_norm|argmax_"
+    names = [n for n in out if re.search(rx, n)]
+    assert len(names) >= 30
+    for n in names:
+        assert len(hits(n)) == 1, (n, hits(n))
