@@ -413,3 +413,72 @@ def test_rocprof_summary_groups_cover_a_batched_profile():
     assert len(names) >= 30
     for n in names:
         assert len(hits(n)) == 1, (n, hits(n))
+
+
+class _CallRecorder:
+    """Stands in for the library: records the sequence that each call addressed."""
+
+    def __init__(self):
+        self.seq, self.calls = 0, []
+
+    def dfl_select_seq(self, ctx, seq):
+        self.seq = seq
+        return 0
+
+    def dfl_cache_reset(self, ctx):
+        self.calls.append(("reset", self.seq))
+        return 0
+
+    def dfl_set_num_layers(self, ctx, n):
+        return 0
+
+    def dfl_last_error(self):
+        return b"refused"
+
+
+def _recorded_model():
+    """A model object without a device: the calls of __call__ up to the kernels' own."""
+    from mirror_sd_amd.dflash import DFlashDraftModel
+
+    class Model(DFlashDraftModel):
+        def __init__(self):
+            self._L, self._ctx = _CallRecorder(), None
+            self.num_draft_layers, self.max_seqs, self._gen, self._batch = 1, 4, 0, 1
+
+        def _ingest(self, th, fused=False):
+            self._L.calls.append(("ingest", self._L.seq))
+            return 1
+
+        def _ingest_seqs(self, th):
+            self._L.calls.append(("ingest_seqs", th.shape[0]))
+            return 1
+
+        def _draft(self, noise=None, **k):
+            self._L.calls.append(("draft", self._L.seq))
+            return noise[0], None, None, None
+
+        def _draft_seqs(self, noise):
+            self._L.calls.append(("draft_seqs", noise.shape[0]))
+            return noise
+
+        def __del__(self):
+            pass
+
+    return Model()
+
+
+def test_call_addresses_the_selected_sequence_and_leaves_sequence_0():
+    """Without a cache, a batch of one runs on the selected sequence, a larger batch on sequences
+    0 .. n-1 whatever was selected; afterwards the single-sequence calls address sequence 0."""
+    import torch
+    x = torch.zeros(1, 2, 4)
+    m = _recorded_model()
+    m.select_seq(2)
+    m(x, x)
+    assert m._L.calls[:3] == [("reset", 2), ("ingest", 2), ("draft", 2)] and m._L.seq == 0
+    m = _recorded_model()
+    m.select_seq(2)
+    x3 = torch.zeros(3, 2, 4)
+    m(x3, x3)
+    assert m._L.calls[:4] == [("reset", 0), ("reset", 1), ("reset", 2), ("ingest_seqs", 3)]
+    assert m._L.seq == 0
