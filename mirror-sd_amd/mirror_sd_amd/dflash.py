@@ -590,12 +590,14 @@ class DFlashDraftModel:
             self._sync_cache(cache, n_seq=B_)
         self._batch = B_
         if cache is None:   # a batch of one: the selected sequence
-            for b in range(B_):
+            try:
+                for b in range(B_):
+                    if B_ > 1:
+                        self.select_seq(b)
+                    _lib.check(self._L.dfl_cache_reset(self._ctx), "dfl_cache_reset")
+            finally:
                 if B_ > 1:
-                    self.select_seq(b)
-                _lib.check(self._L.dfl_cache_reset(self._ctx), "dfl_cache_reset")
-            if B_ > 1:
-                self.select_seq(0)
+                    self.select_seq(0)
         C = self._ingest(target_hidden) if B_ == 1 else self._ingest_seqs(target_hidden)
         if cache is None:
             self._gen += 1

@@ -418,8 +418,8 @@ def test_rocprof_summary_groups_cover_a_batched_profile():
 class _CallRecorder:
     """Stands in for the library: records the sequence that each call addressed."""
 
-    def __init__(self):
-        self.seq, self.calls = 0, []
+    def __init__(self, fail_reset_of=None):
+        self.seq, self.calls, self.fail = 0, [], fail_reset_of
 
     def dfl_select_seq(self, ctx, seq):
         self.seq = seq
@@ -427,7 +427,7 @@ class _CallRecorder:
 
     def dfl_cache_reset(self, ctx):
         self.calls.append(("reset", self.seq))
-        return 0
+        return 3 if self.seq == self.fail else 0
 
     def dfl_set_num_layers(self, ctx, n):
         return 0
@@ -436,13 +436,13 @@ class _CallRecorder:
         return b"refused"
 
 
-def _recorded_model():
+def _recorded_model(**kw):
     """A model object without a device: the calls of __call__ up to the kernels' own."""
     from mirror_sd_amd.dflash import DFlashDraftModel
 
     class Model(DFlashDraftModel):
         def __init__(self):
-            self._L, self._ctx = _CallRecorder(), None
+            self._L, self._ctx = _CallRecorder(**kw), None
             self.num_draft_layers, self.max_seqs, self._gen, self._batch = 1, 4, 0, 1
 
         def _ingest(self, th, fused=False):
@@ -469,7 +469,8 @@ def _recorded_model():
 
 def test_call_addresses_the_selected_sequence_and_leaves_sequence_0():
     """Without a cache, a batch of one runs on the selected sequence, a larger batch on sequences
-    0 .. n-1 whatever was selected; afterwards the single-sequence calls address sequence 0."""
+    0 .. n-1 whatever was selected; afterwards, also after a refused reset, the single-sequence
+    calls address sequence 0."""
     import torch
     x = torch.zeros(1, 2, 4)
     m = _recorded_model()
@@ -481,4 +482,8 @@ def test_call_addresses_the_selected_sequence_and_leaves_sequence_0():
     x3 = torch.zeros(3, 2, 4)
     m(x3, x3)
     assert m._L.calls[:4] == [("reset", 0), ("reset", 1), ("reset", 2), ("ingest_seqs", 3)]
+    assert m._L.seq == 0
+    m = _recorded_model(fail_reset_of=1)
+    with pytest.raises(Exception, match="refused|dfl_cache_reset"):
+        m(x3, x3)
     assert m._L.seq == 0
