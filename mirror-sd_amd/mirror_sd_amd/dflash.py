@@ -167,6 +167,10 @@ class DFlashKVCache:
         return [self.keys, self.values]
 
 
+# Rows of all sequences together up to which dfl_ingest_batch shares one pass (SMALL_ING).
+_STEP_ROWS = 64
+
+
 class DFlashDraftModel:
     """MI355X draft model behind the reference ``DFlashDraftModel`` interface."""
 
@@ -522,10 +526,24 @@ class DFlashDraftModel:
         return C
 
     def _ingest_seqs(self, target_hidden):
-        """Context rows [n_seq, C, nf*H] of sequences 0 .. n_seq-1 (dfl_ingest_batch)."""
+        """Context rows [n_seq, C, nf*H] of sequences 0 .. n_seq-1 (dfl_ingest_batch).  Steps too
+        long to share launches go sequence by sequence where the batch would first have to be
+        copied: the newest rows of a longer buffer are contiguous within a sequence."""
         import torch
+        n_seq, C = target_hidden.shape[0], target_hidden.shape[1]
+        if 2 * C > _STEP_ROWS and not (target_hidden.is_cuda and target_hidden.is_contiguous() and
+                                       target_hidden.dtype == torch.float16):
+            keep = []
+            try:
+                for b in range(n_seq):
+                    self.select_seq(b)
+                    self._ingest(target_hidden[b])
+                    keep.append(self._keep["ingest_src"])
+            finally:
+                self.select_seq(0)
+            self._keep["ingest_src"] = keep
+            return C
         th = target_hidden.to(self.device, torch.float16).contiguous()
-        n_seq, C = th.shape[0], th.shape[1]
         if C == 0:
             return 0
         if th.shape[2] != self.n_feat * self.config.hidden_size:

@@ -76,3 +76,31 @@ def test_batch_rejects(models):
     for args in ((0, p, 1), (MAX_SEQS + 1, p, 1), (2, None, 1), (2, p, -1), (2, p, 100000)):
         m.make_cache(0, 0)
         assert L.dfl_ingest_batch(ctx, *args, None) in (_lib.DFL_EINVAL, _lib.DFL_ERANGE)
+
+
+@pytest.mark.parametrize("n_seq,C", [(3, 70), (2, 33), (3, 20)])
+def test_batch_of_strided_rows(models, n_seq, C):
+    """The newest rows of a longer buffer: the cached rows of a contiguous copy, bit for bit; a
+    step too long to share its launches reads them in place, without a copy of the batch."""
+    a, b = models
+    g = torch.Generator().manual_seed(C)
+    buf = torch.randn((n_seq, 200, 2 * CFG["hidden_size"]), generator=g).to(torch.float16).cuda()
+    th = buf[:, -C:]
+    for m in models:
+        m.make_cache(0, 0)
+        for s in range(MAX_SEQS):
+            m.select_seq(s)
+            _lib.check(m._L.dfl_cache_reset(m._ctx), "dfl_cache_reset")
+        m.select_seq(0)
+    b._ingest_seqs(th.contiguous())
+    torch.cuda.synchronize()
+    a._keep.pop("ingest_src", None)
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    assert a._ingest_seqs(th) == C
+    extra = torch.cuda.max_memory_allocated() - before
+    if 2 * C > 64:
+        assert extra < th.numel() * 2 // n_seq, extra
+    for s in range(n_seq):
+        for (ka, va), (kb, vb) in zip(a.cache_tensors(s), b.cache_tensors(s)):
+            assert torch.equal(ka[:, :C], kb[:, :C]) and torch.equal(va[:, :, :C], vb[:, :, :C])
