@@ -33,7 +33,9 @@ def models():
 
 @pytest.mark.parametrize("ctx,B", [((3, 40), 32), ((1, 31, 97, 500, 2000, 64, 7, 333), 32),
                                    ((9000, 4001, 33), 32), ((5000, 4900, 129, 800), 25),
-                                   ((6001, 3000), 31)])
+                                   ((6001, 3000), 31),
+                                   # 4096 rows (the wide merge) of up to 57 chunks
+                                   ((9000, 40, 33, 7), 32)])
 def test_ring_matches_single(models, ctx, B):
     many, one = models
     g = torch.Generator().manual_seed(sum(ctx))

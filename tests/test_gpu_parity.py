@@ -356,7 +356,8 @@ def test_capacity_boundaries():
                           what=f"layer {layer} values")
 
 
-def test_lm_head_queue_give_up_reports_error_and_recovers():
+@pytest.mark.parametrize("block", [8, 40])   # one and two m-tiles
+def test_lm_head_queue_give_up_reports_error_and_recovers(block):
     """The balanced lm_head's bounded work-queue wait: forced to give up from the host
     (the dfl_test_queue_timeout hook makes its wait condition unsatisfiable for a few
     hundred rounds), every wave still ends, device error bit 2 is set, and the next call --
@@ -365,10 +366,10 @@ def test_lm_head_queue_give_up_reports_error_and_recovers():
     from parity_util import device_errors
     cfg = DFlashConfig(hidden_size=256, num_hidden_layers=1, intermediate_size=512,
                        num_attention_heads=4, num_key_value_heads=2, head_dim=128,
-                       vocab_size=65536, block_size=8, mask_token_id=65535)
+                       vocab_size=65536, block_size=block, mask_token_id=65535)
     t = synth.make_weights_numpy(cfg, seed=5)
-    inp = synth.make_inputs_numpy(cfg, 8, 16, seed=5)
-    m = _model(cfg, max_ctx=16)
+    inp = synth.make_inputs_numpy(cfg, block, 16, seed=5)
+    m = _model(cfg, max_ctx=16, max_block=block)
     m.load_weights(torch_tensors(t, "cuda"))
     ids, lg = m.draft(torch.from_numpy(inp["ids"]), torch.from_numpy(inp["target_hidden"]),
                       return_logits=True)

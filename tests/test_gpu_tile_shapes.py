@@ -99,6 +99,24 @@ def test_append_through_window(model, first, rows):
     _check(model, th, slots, torch.tensor(keep, device="cuda"))
 
 
+@pytest.mark.parametrize("rows", [70, 131])
+def test_wide_hidden_size(rows):
+    """A hidden size above 5120 that is no multiple of 512 (the fc norm's larger register budget,
+    its last step partly past the row)."""
+    from mirror_sd_amd.dflash import DFlashDraftModel
+    cfg = DFlashConfig(hidden_size=5248, num_hidden_layers=1, intermediate_size=512,
+                       num_attention_heads=NKV, num_key_value_heads=NKV, head_dim=128,
+                       vocab_size=512, block_size=8, target_layer_ids=[1], num_target_layers=6)
+    t = torch_tensors(synth.make_weights_numpy(cfg, seed=12), "cuda")
+    m = DFlashDraftModel(cfg, max_ctx=rows)
+    m.load_weights(t)
+    g = torch.Generator().manual_seed(rows)
+    th = torch.randn((rows, 5248), generator=g).to(torch.float16).cuda()
+    m.ingest_seq(0, th)
+    _check((cfg, t, m), th)
+    m.close()
+
+
 def _small(heads, kv, layers, F, **sizes):
     from mirror_sd_amd.dflash import DFlashDraftModel
     cfg = DFlashConfig(hidden_size=H, num_hidden_layers=layers, intermediate_size=F,
