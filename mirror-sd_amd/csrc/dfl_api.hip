@@ -272,7 +272,7 @@ static int setup_ingest(dfl_ctx* x) {
   if ((r = x->alloc(&x->xn, (size_t)x->ing * H)) ||
       (r = x->alloc(&x->ing_cs, (size_t)x->ing * 128)))
     return r;
-  x->fc_ws_floats = x->NF > 0 ? tile_plane_floats(x->ing, H, x->NF * H, WT_F16, x->n_cu) : 0;
+  x->fc_ws_floats = x->NF > 0 ? tile_plane_floats(x->ing, H, x->NF * H, WT_F16, x->n_cu, FC_PLANE_K) : 0;
   if (x->NF > 0 && ((r = x->alloc(&x->fc32, (size_t)x->ing * H)) ||
                     (r = x->alloc(&x->fc_ws, x->fc_ws_floats)) ||
                     (r = x->alloc(&x->xf, (size_t)x->ing * x->NF * H))))
@@ -636,6 +636,7 @@ struct TilePlanes {
   float* ws;
   size_t floats;
   int splits;
+  int plane_k;   // the fewest k of a plane
 };
 static int tgemm(dfl_ctx* ctx, int cat, int wt, int epi, const uint4* W, int N, int K,
                  const half_t* X, int M, const TileArgs& e, hipStream_t st,
@@ -647,7 +648,8 @@ static int tgemm(dfl_ctx* ctx, int cat, int wt, int epi, const uint4* W, int N, 
   // re-tiled last rounds for the epilogues whose outputs do not depend on the tile shape
   // (the ARGMAX keys are per wave column)
   const bool retile = epi != TG_ARGMAX;
-  const TilePlan p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, split_ok, retile, chains);
+  const TilePlan p = tile_plan(M, N, K, wt, ctx->n_cu, epi == TG_SWIGLU, split_ok, retile, chains,
+                               planes && planes->ws ? planes->plane_k : 64);
   if (p.splits > 1 && (size_t)p.splits * M * N > ws_floats)   // (sized for every plan at create)
     return fail(DFL_EINVAL, "tile GEMM: the split-K planes exceed their workspace");
   if (n_parts) *n_parts = N / (32 * p.rbw);
@@ -922,7 +924,7 @@ static int ingest(dfl_ctx* ctx, const uint16_t* src, int C, bool fused, void* st
       // one layer, split against whole: 8B sizes, 65 rows 86 / 160 us, 256 rows 102 / 170, 500
       // rows 145 / 180, from 1000 rows no split; 27B sizes, 65 rows 114 / 238, 256 rows 156 / 271,
       // 777 rows 381 / 400.
-      TilePlanes pl{ctx->fc_ws, ctx->fc_ws_floats, 1};
+      TilePlanes pl{ctx->fc_ws, ctx->fc_ws_floats, 1, FC_PLANE_K};
       DFL_TRY(tgemm(ctx, P_INGEST_FC, WT_F16, TG_F32, ctx->w_fc_pk, H, K, ctx->xf, rows,
                     tile_f32(ctx->fc32, H), st, nullptr, &pl));
       {

@@ -42,6 +42,12 @@ constexpr TileShape kTileShapes[] = {
 // 128, whose few MFMAs a k-block would wait for each other) the halves of the k-blocks
 // alternate between them and the chains are added at the end.
 constexpr int tile_chains(int wt, int mtw, int rbw) { return wt == WT_INT8 && mtw * rbw < 8 ? 2 : 1; }
+// Fewest k of a plane of the ingest's fc, whose planes the norm sums without a launch of its
+// own (the plan counts one): twice what a workgroup's stage buffers hold, as shorter ranges spend
+// their time filling them.  One-layer ingests with planes of at least 1024 / at least 64 k: hidden
+// 2048 (K 10240), 65 rows 50 / 61 us, 128 rows 51 / 63; hidden 1024, 200 rows 40 / 47; hidden 512
+// and 256 (33 / 31, as unsplit) give it up, and keep the sums of the whole product.
+constexpr int FC_PLANE_K = 1024;
 constexpr int kNumTileShapes = (int)(sizeof(kTileShapes) / sizeof(kTileShapes[0]));
 
 // The 4-wave shapes add four loader waves that issue every global -> LDS copy (the compute
@@ -86,8 +92,10 @@ constexpr int tile_stages(int wt, int wm, int mtw, int rbw, int wn, int kc) {
 // chains (optional): only shapes with that many accumulation chains, so that a product's sums
 // are those of another plan (unsplit sums depend on the chains alone).
 // pairs: each wave must hold gate|up row-block pairs (SWIGLU), i.e. an even rbw.
+// plane_k: the fewest k of a split-K plane.
 inline TilePlan tile_plan(int M, int N, int K, int wt, int n_cu, bool pairs = false,
-                          bool split = false, bool retile = false, int chains = 0) {
+                          bool split = false, bool retile = false, int chains = 0,
+                          int plane_k = 64) {
   TilePlan best{};
   double best_t = 1e300;
   for (const TileShape& s : kTileShapes) {
@@ -97,7 +105,7 @@ inline TilePlan tile_plan(int M, int N, int K, int wt, int n_cu, bool pairs = fa
     const int bm = 32 * s.wm * s.mtw, bn = 32 * s.rbw * s.wn;
     if (N % bn) continue;
     const long long tiles = (long long)((M + bm - 1) / bm) * (N / bn);
-    for (int sp = 1; sp <= (split ? 16 : 1) && sp <= K / 64; sp *= 2) {
+    for (int sp = 1; sp <= (split ? 16 : 1) && sp * plane_k <= std::max(K, plane_k); sp *= 2) {
       if (sp > 1 && tiles * sp > n_cu) break;
       const long long full = tiles * sp / n_cu, part = tiles * sp % n_cu;
       const double rounds =
@@ -153,10 +161,10 @@ inline TilePlan tile_plan(int M, int N, int K, int wt, int n_cu, bool pairs = fa
 // RESID product with re-tiled last rounds): the most over every row count, as neither the factor
 // nor the planes grow evenly with the rows.  A workspace of this size holds every plan, so that
 // a product's split, and with it the order of its sums, is a rule on the product alone.
-inline size_t tile_plane_floats(int rows, int N, int K, int wt, int n_cu) {
+inline size_t tile_plane_floats(int rows, int N, int K, int wt, int n_cu, int plane_k = 64) {
   size_t most = 0;
   for (int M = 1; M <= rows; ++M) {
-    const TilePlan p = tile_plan(M, N, K, wt, n_cu, false, true, true);
+    const TilePlan p = tile_plan(M, N, K, wt, n_cu, false, true, true, 0, plane_k);
     if (p.splits > 1) most = std::max(most, (size_t)p.splits * M * N);
   }
   return most;
