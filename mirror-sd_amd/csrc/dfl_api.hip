@@ -525,9 +525,9 @@ int dfl_load_head(dfl_ctx* ctx, const uint16_t* final_norm, const uint16_t* embe
   return DFL_OK;
 }
 
-// Stream-K GEMM over the M rows of a block: one 32-row m-tile per launch of the
-// single-tile kernel, or two per launch of the two-tile kernel (each weight block read
-// once for both).  A normed input (gnorm set) takes its 1/rms rows from
+// Stream-K GEMM over the M rows of a block or a per-step ingest, up to 32 (the single-tile
+// kernel) or 64 (the two-tile kernel: each weight block read once for both m-tiles).  A normed
+// input (gnorm set) takes its 1/rms rows from
 // the embedding kernel (rn_from_ss false) or from the row sums of squares that the
 // previous RESID GEMM left in sk_ss (rn_from_ss true).
 static int skgemm(dfl_ctx* ctx, int cat, int wt, int epi, const SKPlan& p,
@@ -539,71 +539,65 @@ static int skgemm(dfl_ctx* ctx, int cat, int wt, int epi, const SKPlan& p,
                    const FeatPtrs* xr = nullptr, int xr_h = 0) {
   const long long wbytes = (wt == WT_INT8) ? (long long)N * KB * 32 + 2LL * N
                                            : (long long)N * KB * 16 * 2;
-  const int ss_stride = (ctx->H / 64) * 32;
-  const int n_mt = (M + 31) / 32;
-  for (int g0 = 0; g0 < n_mt; g0 += MT_MAX) {
-    const int mt_n = std::min(MT_MAX, n_mt - g0);
-    const int m0 = g0 * 32;
-    ProfScope ps(ctx, cat, wbytes, st, /*attached=*/true);
-    StreamArgs a{};
-    a.W = W;
-    a.scale = scale;
-    a.N = N;
-    a.KB = KB;
-    a.X = X ? X + (size_t)m0 * ldx : nullptr;
-    a.ldx = ldx;
-    if (xr) {   // row-major feature rows read in place (one m-tile)
-      a.xr_n = xr->n;
-      a.xr_ld = xr->ld;
-      a.xr_h = xr_h;
-      for (int j = 0; j < xr->n; ++j) a.xr_p[j] = xr->p[j];
-    }
-    a.M = std::min(32 * mt_n, M - m0);
-    a.MT = mt_n;
-    a.rnorm = ctx->rnorm + m0;
-    a.ss_in = rn_from_ss ? ctx->sk_ss + (size_t)g0 * ss_stride : nullptr;
-    a.ss_tiles = ctx->H / 64;
-    a.ss_n = ctx->H;
-    a.ss_mstride = ss_stride;
-    a.gnorm = gnorm;
-    a.ws = ctx->sk_ws;
-    // the hybrid plan when it has whole tiles per workgroup; the fused qkv kernel (a Q/K
-    // head's two tiles complete together) keeps the contiguous partition
-    a.dp = streamk_launch_dp(p, epi, false);
-    // test hook of the balanced kernel's bounded work-queue wait (its give-up path), set
-    // only through dfl_test_queue_timeout
-    a.dyn_test_timeout = p.dyn_static > 0 && ctx->test_queue_timeout;
-    a.seg_cap = a.dp > 0 ? p.sk_seg_cap : p.seg_cap;
-    a.tile_cnt = ctx->sk_tile_cnt;
-    a.out = out ? out + (size_t)m0 * ldo : nullptr;
-    a.ldo = ldo;
-    a.x = xres ? xres + (size_t)m0 * ldo : nullptr;
-    a.x_zero = x_zero;
-    a.ss_part = ctx->sk_ss + (size_t)g0 * ss_stride;
-    a.eps = ctx->cfg.rms_eps;
-    a.logits = logits ? logits + (size_t)m0 * N : nullptr;
-    a.ldl = N;
-    a.keys = keys ? keys + m0 : nullptr;
-    a.dyn_static = p.dyn_static;
-    a.dyn_next = ctx->dyn_next;
-    a.err = ctx->err;
-    if (epi == EPI_ARGMAX) {
-      a.samp_invT = ctx->call_invT;
-      a.samp_seed = ctx->call_seed;
-      a.samp_row0 = m0;
-    }
-    // the balanced kernel finalises the argmax ids of its rows itself
-    const bool fin = ids && keys && p.dyn_static > 0 && n_mt <= MT_MAX;
-    a.ids = fin ? ids : nullptr;
-    if (ids_done) *ids_done = fin;
-    if (rope) a.rope = *rope;
-    if (const char* why = check_stream_args(wt, epi, gnorm != nullptr, a, p, mt_n > 1))
-      return fail(DFL_EINVAL, std::string("stream-K GEMM launch refused: ") + why);
-    const bool ok =
-        mt_n == 1 ? launch_streamk_gemm(wt, epi, gnorm != nullptr, a, p, st, ps.start(), ps.stop())
-                  : launch_streamk_gemm_m(wt, epi, gnorm != nullptr, a, p, st, ps.start(), ps.stop());
-    if (!ok) return fail(DFL_EINVAL, "no GEMM kernel for this weight type / epilogue");
+  const int n_mt = (M + 31) / 32;   // 1 or 2: more rows are refused below
+  ProfScope ps(ctx, cat, wbytes, st, /*attached=*/true);
+  StreamArgs a{};
+  a.W = W;
+  a.scale = scale;
+  a.N = N;
+  a.KB = KB;
+  a.X = X;
+  a.ldx = ldx;
+  if (xr) {   // row-major feature rows read in place (one m-tile)
+    a.xr_n = xr->n;
+    a.xr_ld = xr->ld;
+    a.xr_h = xr_h;
+    for (int j = 0; j < xr->n; ++j) a.xr_p[j] = xr->p[j];
   }
+  a.M = M;
+  a.MT = n_mt;
+  a.rnorm = ctx->rnorm;
+  a.ss_in = rn_from_ss ? ctx->sk_ss : nullptr;
+  a.ss_tiles = ctx->H / 64;
+  a.ss_n = ctx->H;
+  a.ss_mstride = (ctx->H / 64) * 32;
+  a.gnorm = gnorm;
+  a.ws = ctx->sk_ws;
+  // the hybrid plan when it has whole tiles per workgroup; the fused qkv kernel (a Q/K
+  // head's two tiles complete together) keeps the contiguous partition
+  a.dp = streamk_launch_dp(p, epi);
+  // test hook of the balanced kernel's bounded work-queue wait (its give-up path), set
+  // only through dfl_test_queue_timeout
+  a.dyn_test_timeout = p.dyn_static > 0 && ctx->test_queue_timeout;
+  a.seg_cap = a.dp > 0 ? p.sk_seg_cap : p.seg_cap;
+  a.tile_cnt = ctx->sk_tile_cnt;
+  a.out = out;
+  a.ldo = ldo;
+  a.x = xres;
+  a.x_zero = x_zero;
+  a.ss_part = ctx->sk_ss;
+  a.eps = ctx->cfg.rms_eps;
+  a.logits = logits;
+  a.ldl = N;
+  a.keys = keys;
+  a.dyn_static = p.dyn_static;
+  a.dyn_next = ctx->dyn_next;
+  a.err = ctx->err;
+  if (epi == EPI_ARGMAX) {
+    a.samp_invT = ctx->call_invT;
+    a.samp_seed = ctx->call_seed;
+  }
+  // the balanced kernel finalises the argmax ids itself
+  const bool fin = ids && keys && p.dyn_static > 0;
+  a.ids = fin ? ids : nullptr;
+  if (ids_done) *ids_done = fin;
+  if (rope) a.rope = *rope;
+  if (const char* why = check_stream_args(wt, epi, gnorm != nullptr, a, p, n_mt > 1))
+    return fail(DFL_EINVAL, std::string("stream-K GEMM launch refused: ") + why);
+  const bool ok =
+      n_mt == 1 ? launch_streamk_gemm(wt, epi, gnorm != nullptr, a, p, st, ps.start(), ps.stop())
+                : launch_streamk_gemm_m(wt, epi, gnorm != nullptr, a, p, st, ps.start(), ps.stop());
+  if (!ok) return fail(DFL_EINVAL, "no GEMM kernel for this weight type / epilogue");
   return DFL_OK;
 }
 

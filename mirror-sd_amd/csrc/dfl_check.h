@@ -13,14 +13,14 @@ constexpr int CHECK_WG_WAVES = 4;   // streaming waves of a stream-K workgroup (
 constexpr int CHECK_MAX_CHUNKS = 64;
 
 inline const char* check_stream_args(int wt, int epi, bool norm, const StreamArgs& a,
-                                     const SKPlan& p, bool m_split) {
+                                     const SKPlan& p, bool two_tile) {
   if (wt != WT_INT8 && wt != WT_F16) return "unknown weight type";
   if (!a.W) return "null weight matrix";
   if (a.N <= 0 || a.N % 64) return "N must be a positive multiple of 64";
   if (a.KB < CHECK_WG_WAVES) return "fewer k-blocks than streaming waves";
   if (a.xr_n < 0 || a.xr_n > MAX_FEATS) return "row-major activations: feature count out of range";
   if (a.xr_n > 0) {
-    if (wt != WT_F16 || epi != EPI_RESID || norm || m_split)
+    if (wt != WT_F16 || epi != EPI_RESID || norm || two_tile)
       return "row-major activations are read by the one-tile fp16 RESID kernel only";
     if (a.xr_h < 64 || a.xr_h % 16 || (long long)a.xr_n * a.xr_h != (long long)a.KB * 16)
       return "row-major activations: features do not tile the K axis in 16-column blocks";
@@ -33,7 +33,7 @@ inline const char* check_stream_args(int wt, int epi, bool norm, const StreamArg
     return "null activations";
   }
   if (a.M < 1) return "no activation rows";
-  if (m_split ? (a.MT != 2 || a.M > 32 * a.MT) : (a.M > 32))
+  if (two_tile ? (a.MT != 2 || a.M > 32 * a.MT) : (a.M > 32))
     return "activation rows exceed the kernel's m-tiles";
   if (p.workers < 1 || a.seg_cap < 1 || !a.ws || !a.tile_cnt)
     return "missing split-tile workspace";
@@ -60,7 +60,7 @@ inline const char* check_stream_args(int wt, int epi, bool norm, const StreamArg
       break;
     case EPI_QKROPE: {
       const RopeEpi& r = a.rope;
-      if (m_split || a.M > 32 || !norm) return "QKROPE is the single-tile normed qkv kernel";
+      if (two_tile || a.M > 32 || !norm) return "QKROPE is the single-tile normed qkv kernel";
       if (a.N != (r.NH + 2 * r.NKV) * 128 || r.NH < 1 || r.NKV < 1)
         return "QKROPE rows are not the q|k|v heads";
       if (a.N > QK_N_MAX) return "QKROPE: more q|k|v rows than the scales' LDS copy holds";

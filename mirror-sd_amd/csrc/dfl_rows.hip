@@ -755,7 +755,6 @@ static_assert(SA_LISTS * SA_TOPK_MAX * 8 % 16 == 0 && SA_LISTS <= EB_THREADS, "c
 // counting), then sums the k rows with every row's load in flight.  Latency-bound: 151936 bf16
 // logits, H = 4096, 16 rows: both launches 15.2 us, against 40.8 with per-thread lists popped
 // through LDS and barriers and one row's element load at a time.
-template <int DT>
 __global__ __launch_bounds__(EB_THREADS) void embed_block_kernel(
     const int32_t* __restrict__ ids, const half_t* __restrict__ embed, int Vemb, int H,
     bool anchor, int k, const unsigned long long* __restrict__ cand, half_t* __restrict__ out,
@@ -865,7 +864,7 @@ static void launch_embed_block_t(const int32_t* ids, int B, const half_t* embed,
   if (logits)
     hipLaunchKernelGGL(topk_scan_kernel<DT>, dim3(SA_BLOCKS), dim3(64 * SA_WAVES), 0, st, logits,
                        V, top_k, cand);
-  hipLaunchKernelGGL(embed_block_kernel<DT>, dim3(B), dim3(EB_THREADS), 0, st, ids, embed, Vemb, H,
+  hipLaunchKernelGGL(embed_block_kernel, dim3(B), dim3(EB_THREADS), 0, st, ids, embed, Vemb, H,
                      logits != nullptr, top_k, cand, out, err, vec);
 }
 

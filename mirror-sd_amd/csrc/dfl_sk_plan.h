@@ -51,10 +51,9 @@ inline SKPlan streamk_plan_balanced(int N, int KB, int n_cu) {
 
 // Whole tiles per workgroup that one launch of plan p uses.  The fused qkv kernel
 // (EPI_QKROPE: a Q/K head's two tiles complete together, worker counts taken from the
-// contiguous partition) and a launch that splits the m-tiles over the waves (m_split; none
-// does any more) keep the contiguous partition.
-inline int streamk_launch_dp(const SKPlan& p, int epi, bool m_split) {
-  return (!m_split && epi != EPI_QKROPE) ? p.dp : 0;
+// contiguous partition) keeps the contiguous partition.
+inline int streamk_launch_dp(const SKPlan& p, int epi) {
+  return epi != EPI_QKROPE ? p.dp : 0;
 }
 
 }  // namespace dfl

@@ -496,7 +496,7 @@ bool launch_shape_i(int wt, int epi, const TileArgs& a, const TilePlan& p, hipSt
   if constexpr (I < kNumTileShapes) {
     constexpr TileShape s = kTileShapes[I];
     if (wt == s.wt && (shape >= 0 ? shape == I
-                                  : (!s.tail && p.wm == s.wm && p.mtw == s.mtw && p.rbw == s.rbw &&
+                                  : (p.wm == s.wm && p.mtw == s.mtw && p.rbw == s.rbw &&
                                      p.wn == s.wn && p.kc == s.kc))) {
       if (epi == TG_F32) {
         launch_tile<s.wt, TG_F32, s.wm, s.mtw, s.rbw, s.wn, s.kc>(a, st, e0, e1);

@@ -23,20 +23,18 @@ constexpr int TG_LDS_BUDGET = 160 * 1024;  // one workgroup per CU
 // 5120 against 494 with four rows of 1 x 4, and 128 x 64 in 560 against 593; the 256 x 128
 // wave hides it under its MFMAs (375 us).  256 x 256 was slower in every arrangement (416-440).
 // fp16, 777 x 4096 x 20480: 128 x 128 166 us, 256 x 64 225.
-// tail: used only to re-tile the partial last round of a larger shape's plan.
 struct TileShape {
   int wt, wm, mtw, rbw, wn, kc, cyc;
-  bool tail;
 };
 constexpr TileShape kTileShapes[] = {
-    {WT_INT8, 4, 1, 1, 1, 64, 410, false},    // 128 x 32
-    {WT_INT8, 2, 2, 1, 2, 64, 450, false},    // 128 x 64
-    {WT_INT8, 2, 2, 2, 2, 64, 690, false},    // 128 x 128
-    {WT_INT8, 4, 2, 4, 1, 64, 1100, false},   // 256 x 128
-    {WT_F16, 4, 2, 2, 1, 64, 860, false},     // 256 x 64
-    {WT_F16, 4, 1, 4, 1, 64, 680, false},     // 128 x 128
-    {WT_F16, 4, 2, 4, 1, 32, 1200, false},    // 256 x 128
-    {WT_F16, 4, 2, 4, 2, 32, 2200, false},    // 256 x 256
+    {WT_INT8, 4, 1, 1, 1, 64, 410},    // 128 x 32
+    {WT_INT8, 2, 2, 1, 2, 64, 450},    // 128 x 64
+    {WT_INT8, 2, 2, 2, 2, 64, 690},    // 128 x 128
+    {WT_INT8, 4, 2, 4, 1, 64, 1100},   // 256 x 128
+    {WT_F16, 4, 2, 2, 1, 64, 860},     // 256 x 64
+    {WT_F16, 4, 1, 4, 1, 64, 680},     // 128 x 128
+    {WT_F16, 4, 2, 4, 1, 32, 1200},    // 256 x 128
+    {WT_F16, 4, 2, 4, 2, 32, 2200},    // 256 x 256
 };
 // Independent MFMA accumulation chains of an output block: with two (int8 tiles of up to 128 x
 // 128, whose few MFMAs a k-block would wait for each other) the halves of the k-blocks
@@ -99,7 +97,7 @@ inline TilePlan tile_plan(int M, int N, int K, int wt, int n_cu, bool pairs = fa
   TilePlan best{};
   double best_t = 1e300;
   for (const TileShape& s : kTileShapes) {
-    if (s.tail || s.wt != wt || K % s.kc || (pairs && s.rbw % 2) ||
+    if (s.wt != wt || K % s.kc || (pairs && s.rbw % 2) ||
         (chains && tile_chains(wt, s.mtw, s.rbw) != chains))
       continue;
     const int bm = 32 * s.wm * s.mtw, bn = 32 * s.rbw * s.wn;

@@ -86,15 +86,14 @@ int main() {
         StreamArgs b = r;
         b.rope.NH = hk[0]; b.rope.NKV = hk[1]; b.N = (hk[0] + 2 * hk[1]) * 128;
         const SKPlan sp = streamk_plan(b.N, b.KB, ncu);
-        b.dp = streamk_launch_dp(sp, EPI_QKROPE, false);
+        b.dp = streamk_launch_dp(sp, EPI_QKROPE);
         b.seg_cap = b.dp > 0 ? sp.sk_seg_cap : sp.seg_cap;
         char what[96];
         std::snprintf(what, sizeof what, "QKROPE launch %d/%d heads on %d CUs", hk[0], hk[1], ncu);
         if (b.dp != 0) expect("dp > 0", nullptr, what);
         expect(check_stream_args(WT_INT8, EPI_QKROPE, true, b, sp, false), nullptr, what);
         // the other epilogues take the hybrid plan whenever it has whole tiles
-        if (streamk_launch_dp(sp, EPI_STORE, false) != sp.dp) expect("store dp", nullptr, what);
-        if (streamk_launch_dp(sp, EPI_STORE, true) != 0) expect("m-split dp", nullptr, what);
+        if (streamk_launch_dp(sp, EPI_STORE) != sp.dp) expect("store dp", nullptr, what);
       }
     { StreamArgs b = r; b.dp = 1; SKPlan sp = streamk_plan(7168, 160, 64); b.seg_cap = sp.sk_seg_cap;
       expect(check_stream_args(WT_INT8, EPI_QKROPE, true, b, sp, false), "QKROPE", "QKROPE with dp > 0"); }
@@ -219,18 +218,10 @@ int main() {
       q = rt; q.tail_shape = kNumTileShapes;
       expect(check_tile_args(WT_F16, TG_F32, b, q), "unknown", "re-tiled shape index"); }
     // none without permission, nor when the tiles fill whole rounds (K|V ingest: 16 x 16
-    // tiles of 256 x 128), nor in the plain plan's shape list
+    // tiles of 256 x 128)
     if (tile_plan(4096, 5120, 25600, WT_F16, 256).tail_shape != -1) expect("tail", nullptr, "fc no re-tile");
     if (tile_plan(4096, 2048, 5120, WT_INT8, 256, false, false, true).tail_shape != -1)
       expect("tail", nullptr, "K|V whole rounds");
-    for (int M : {256, 1024, 4096})
-      for (int N : {5120, 28672, 128256}) {
-        const TilePlan q = tile_plan(M, N, 5120, WT_F16, 256);
-        for (const TileShape& u : kTileShapes)
-          if (u.tail && u.wt == WT_F16 && q.mtw == u.mtw && q.rbw == u.rbw && q.wn == u.wn &&
-              q.kc == u.kc)
-            expect("tail-only shape planned", nullptr, "plain plan shapes");
-      }
   }
   if (fails == 0) std::printf("ok\n");
   return fails ? 1 : 0;
