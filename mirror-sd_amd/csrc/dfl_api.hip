@@ -157,9 +157,8 @@ struct dfl_ctx {
   SKPlan sk_qkv, sk_o, sk_gu, sk_down, sk_lm;
   // context ingest: `ing` rows per pass (compute-bound: fc and K|V on the tile GEMM)
   int ing = 0;
-  float* fc32 = nullptr;      // [ing][H] fc GEMM rows (fp32)
-  float* fc_ws = nullptr;     // split-K planes of the fc product, of any row count up to ing
-  size_t fc_ws_floats = 0;
+  float* fc32 = nullptr;      // [ing][H] fc GEMM rows (fp32), or their split-K planes, which have
+  size_t fc32_floats = 0;     // room here at any row count up to ing
   float* ing_cs = nullptr;    // [ing][64][2] RoPE (cos, sin) of a prompt-sized pass's rows
   half_t* xf = nullptr;       // [ing][n_target_feat * H] fc input rows, fragment layout
   half_t* xn = nullptr;       // [ing/32][32][H] hidden_norm(fc) (or fused) rows, fragment layout
@@ -272,11 +271,13 @@ static int setup_ingest(dfl_ctx* x) {
   if ((r = x->alloc(&x->xn, (size_t)x->ing * H)) ||
       (r = x->alloc(&x->ing_cs, (size_t)x->ing * 128)))
     return r;
-  x->fc_ws_floats = x->NF > 0 ? tile_plane_floats(x->ing, H, x->NF * H, WT_F16, x->n_cu, FC_PLANE_K) : 0;
-  if (x->NF > 0 && ((r = x->alloc(&x->fc32, (size_t)x->ing * H)) ||
-                    (r = x->alloc(&x->fc_ws, x->fc_ws_floats)) ||
-                    (r = x->alloc(&x->xf, (size_t)x->ing * x->NF * H))))
-    return r;
+  if (x->NF > 0) {
+    x->fc32_floats = std::max(
+        (size_t)x->ing * H, tile_plane_floats(x->ing, H, x->NF * H, WT_F16, x->n_cu, FC_PLANE_K));
+    if ((r = x->alloc(&x->fc32, x->fc32_floats)) ||
+        (r = x->alloc(&x->xf, (size_t)x->ing * x->NF * H)))
+      return r;
+  }
   return DFL_OK;
 }
 
@@ -918,13 +919,13 @@ static int ingest(dfl_ctx* ctx, const uint16_t* src, int C, bool fused, void* st
       // one layer, split against whole: 8B sizes, 65 rows 86 / 160 us, 256 rows 102 / 170, 500
       // rows 145 / 180, from 1000 rows no split; 27B sizes, 65 rows 114 / 238, 256 rows 156 / 271,
       // 777 rows 381 / 400.
-      TilePlanes pl{ctx->fc_ws, ctx->fc_ws_floats, 1, FC_PLANE_K};
+      TilePlanes pl{ctx->fc32, ctx->fc32_floats, 1, FC_PLANE_K};
       DFL_TRY(tgemm(ctx, P_INGEST_FC, WT_F16, TG_F32, ctx->w_fc_pk, H, K, ctx->xf, rows,
                     tile_f32(ctx->fc32, H), st, nullptr, &pl));
       {
         ProfScope ps(ctx, P_INGEST_FC, 0, st);
-        launch_fc_norm_rows(pl.splits > 1 ? ctx->fc_ws : ctx->fc32, pl.splits, rows, H,
-                            ctx->hidden_norm, ctx->cfg.rms_eps, ctx->xn, st);
+        launch_fc_norm_rows(ctx->fc32, pl.splits, rows, H, ctx->hidden_norm, ctx->cfg.rms_eps,
+                            ctx->xn, st);
       }
       DFL_TRY(ingest_kv_rows(ctx, ctx->xn, rows, r0, st));
     }
