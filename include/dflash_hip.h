@@ -94,8 +94,11 @@ int dfl_load_head(dfl_ctx* ctx, const uint16_t* final_norm, const uint16_t* embe
  * `_compute_context`, ane_model.py:632-637).  target_hidden [C][n_target_feat*H] fp16. */
 int dfl_ingest_context(dfl_ctx* ctx, const uint16_t* target_hidden, int32_t C, void* stream);
 /* The same for sequences 0 .. n_seq-1 in lockstep, C rows each: target_hidden
- * [n_seq][C][n_target_feat*H].  Short steps of several sequences share one pass over the
- * fc and K/V weights; each sequence's rows are those of its own dfl_ingest_context call. */
+ * [n_seq][C][n_target_feat*H].  Steps of at most 64 rows in all (and 8 sequences) share one
+ * pass over the fc and K/V weights, larger ones go in such groups or sequence by sequence.  The
+ * kernels, and with them the order of the fp32 sums, follow the rows of a group: a sequence's
+ * rows agree with its own dfl_ingest_context call to the fp16 rounding of those sums, not bit
+ * for bit. */
 int dfl_ingest_batch(dfl_ctx* ctx, int32_t n_seq, const uint16_t* target_hidden, int32_t C,
                      void* stream);
 /* Same for context rows that are already fused ([C][H] fp16): skips fc + hidden_norm. */
@@ -211,7 +214,7 @@ int dfl_embed_block(dfl_ctx* ctx, const int32_t* ids, int32_t B, const void* cor
  * that receives the same error bits as dfl_device_errors (OR'ed in; bit 0 a token id outside
  * [0, Vemb), bit 1 soft-anchor logits without a single number).  Other arguments, checks and
  * results as dfl_embed_block.  The soft anchor's top-k candidates go to a fixed 16 KiB device
- * array of the library (64 scan workgroups x 8 keys, one copy per GPU, held until the process
+ * array of the library (256 scan waves x 8 keys, one copy per GPU, held until the process
  * ends), so the call allocates nothing; concurrent calls on one GPU share that array and
  * race, so a caller serialises them (one stream, or events between streams). */
 int dfl_embed_block_noalloc(const int32_t* ids, int32_t B, const uint16_t* embed, int32_t Vemb,

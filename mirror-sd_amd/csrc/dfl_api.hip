@@ -137,7 +137,7 @@ struct dfl_ctx {
   half_t *x = nullptr, *h = nullptr, *Q = nullptr, *attn = nullptr, *act = nullptr;
   float *Op = nullptr, *Ml = nullptr;
   unsigned long long* keys = nullptr;
-  unsigned long long* sa_cand = nullptr;   // soft-anchor top-k candidates per scan workgroup
+  unsigned long long* sa_cand = nullptr;   // soft-anchor top-k candidates per scan wave
   int* err = nullptr;
   // stream-K GEMM state (block step)
   int n_cu = 256;
@@ -916,9 +916,9 @@ static int ingest(dfl_ctx* ctx, const uint16_t* src, int C, bool fused, void* st
       // Few rows leave CUs without a tile: the product may then split its long K into fp32
       // planes, which the norm sums.  The planes have room of their own for every row count, so
       // the same rows get the same sums whatever the model's max_ctx and layers.  Ingests of
-      // one layer, split against whole: 8B sizes, 65 rows 86 / 160 us, 256 rows 102 / 170, 500
-      // rows 145 / 180, from 1000 rows no split; 27B sizes, 65 rows 114 / 238, 256 rows 156 / 271,
-      // 777 rows 381 / 400.
+      // one layer, split against whole: 8B sizes, 65 rows 83 / 160 us, 256 rows 99 / 170, 500
+      // rows 144 / 180, from 1000 rows no split; 27B sizes, 65 rows 114 / 238, 256 rows 155 / 271,
+      // 777 rows 382 / 388.
       TilePlanes pl{ctx->fc32, ctx->fc32_floats, 1, FC_PLANE_K};
       DFL_TRY(tgemm(ctx, P_INGEST_FC, WT_F16, TG_F32, ctx->w_fc_pk, H, K, ctx->xf, rows,
                     tile_f32(ctx->fc32, H), st, nullptr, &pl));
@@ -1192,7 +1192,9 @@ static int draft_rows(dfl_ctx* ctx, const char* who, int seq0, int n_seq,
         as.sink_len = std::min(after.len, after.sink);
         // every key in range valid (the ring full, or never wrapped): no key needs the mask, so
         // the kernel takes the unmasked softmax (a ring position costs a modulo a key: 1088 keys,
-        // 27B-class heads, 16.3 -> 10.3 us)
+        // 27B-class heads, 16.3 -> 10.3 us).  The two softmaxes round differently (the unmasked
+        // one scales and subtracts in one fma): a layer's hidden states differ by 4e-4 of their
+        // norm, each 1.1e-3 off the 64-bit result
         if (as.L <= after.sink ? as.sink_len == as.L
                                : as.sink_len == after.sink && as.ring_len == as.L - after.sink)
           as.ring_W = 0;

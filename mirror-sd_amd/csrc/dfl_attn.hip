@@ -427,10 +427,13 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(AttnArgs a) {
 }
 
 // The same with half a wave per row and 16 bytes a lane and chunk (a quarter of the load
-// instructions, no barrier), in the same order of sums: 8192 rows of up to 13 chunks 9.7 us
-// against 12.9; but fewer waves to hide the loads behind, 1280 rows of 26 chunks 6.5 against 5.0.
+// instructions, no barrier), in the same order of sums, but with fewer waves to hide the loads
+// behind.  us, wide / narrow, at 500 and 8000 keys of context (32 or 40 heads over 8): 1024 rows
+// 6.0 / 5.0 and 7.2 / 5.2, 2048 rows 7.0 / 5.6 and 9.0 / 8.3, 3072 rows (three sequences) 9.0 / 7.7
+// and 8.3 / 8.2, 3840 rows 9.2 / 9.3 and 9.4 / 9.9, 4096 rows 6.2 / 7.5 and 8.5 / 8.8 (one
+// sequence 9.6 / 9.8 and 13.1 / 13.8), 8192 rows 7.8 / 10.4 and 9.1 / 11.8.
 constexpr int MERGE_WIDE_ROWS = 8;      // rows per workgroup
-constexpr int MERGE_WIDE_MIN = 4096;    // rows from which a launch uses it
+constexpr int MERGE_WIDE_MIN = 4096;    // rows from which a launch uses it (they cross at 3072-3840)
 __global__ __launch_bounds__(32 * MERGE_WIDE_ROWS) void attn_merge_wide_kernel(AttnArgs a,
                                                                                int n_rows) {
   __shared__ float wts[MERGE_WIDE_ROWS][64];
@@ -511,7 +514,10 @@ bool launch_block_attention(const AttnArgs& a_in, hipStream_t st) {
   const bool pipe = a.n_seq == 1 && a.sq[0].chunk > 32 * AT_STAGE_BLOCKS && a.kw == 1 &&
                     a.q_per_group <= 5 && (long long)a.chunk0[1] * a.NKV * groups <= a.n_cu &&
                     a.lds_max >= 2 * AT_STAGE_BYTES;
-  // (a wave takes every key block of its tile in order, so the sums are the single buffer's)
+  // (a wave takes every key block of its tile in order, so the sums are the single buffer's).
+  // Four tiles only: the ring's counted waits take a block's 16 segments as four loads of each of
+  // four waves.  Launches of other widths keep the single buffer; a ring for three or five waves,
+  // whose shares differ, was not built, and what it would give is not measured.
   const bool ring = a.n_seq > 1 && a.kw == 1 && a.q_per_group == 4;
   const dim3 grid(a.chunk0[a.n_seq], a.NKV, groups), block(64 * a.q_per_group * a.kw);
   if (pipe && a.q_per_group == 5)

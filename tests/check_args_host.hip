@@ -61,7 +61,7 @@ int main() {
     { StreamArgs b = r; b.xr_n = MAX_FEATS + 1; expect(check_stream_args(WT_F16, EPI_RESID, false, b, p, false), "count", "xr_n range"); }
     { StreamArgs b = r; expect(check_stream_args(WT_F16, EPI_STORE, false, b, p, false), "one-tile fp16 RESID", "row-major STORE"); }
     { StreamArgs b = r; expect(check_stream_args(WT_F16, EPI_RESID, true, b, p, false), "one-tile fp16 RESID", "row-major norm"); }
-    { StreamArgs b = r; b.M = 64; b.MT = 2; expect(check_stream_args(WT_F16, EPI_RESID, false, b, p, true), "one-tile fp16 RESID", "row-major m-split"); }
+    { StreamArgs b = r; b.M = 64; b.MT = 2; expect(check_stream_args(WT_F16, EPI_RESID, false, b, p, true), "one-tile fp16 RESID", "row-major two-tile"); }
     { StreamArgs b = r; b.xr_h = 5112; expect(check_stream_args(WT_F16, EPI_RESID, false, b, p, false), "tile the K axis", "xr_h % 16"); }
     { StreamArgs b = r; b.xr_n = 4; expect(check_stream_args(WT_F16, EPI_RESID, false, b, p, false), "tile the K axis", "features short of K"); }
     { StreamArgs b = r; b.xr_ld = 5116; expect(check_stream_args(WT_F16, EPI_RESID, false, b, p, false), "row stride", "xr_ld"); }

@@ -1,6 +1,6 @@
 """RMSNorm gains that differ from column to column (a trained model's; the synthetic weights of
 the other tests have unit gains) through every kernel that applies a norm as it loads its
-input: the stream-K projections and lm_head of one block, the M-split projections of stacked
+input: the stream-K projections and lm_head of one block, the two-m-tile projections of stacked
 rows, and the per-step ingest's K|V projection.  Against the CPU oracle, with the tolerance of
 the other draft tests (cosine >= 0.9995, max-abs <= 2e-2 in fp16)."""
 
